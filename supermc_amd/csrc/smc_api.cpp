@@ -195,6 +195,7 @@ struct smc_ctx {
   unsigned* kln_list = nullptr;   // active cells of the per-cell quadrature (an event chunk), then its count
   int kln_npt = 0, kln_nn = 0;
   KlnConst kln_kc{};
+  KlnBreaks kln_breaks{};         // breakpoint tables of the per-cell quadrature (first use)
   // differentiable batches
   DiffBufs dif{};
   void* dif_alloc[16] = {};
@@ -730,6 +731,25 @@ void ensure_kln_table(smc_ctx* c) {
   (void)hipFree(db);
 }
 
+// The breakpoint tables of the per-cell quadrature, built on its first use;
+// node tables they do not fit stay on the node-by-node kernel.
+void ensure_kln_breaks(smc_ctx* c) {
+  KlnBreaks& kb = c->kln_breaks;
+  if (kb.tab || !kln_breaks_fit(c->kln_npt, c->kln_nn)) return;
+  const size_t nb = (size_t)c->kln_npt * (c->kln_nn + 1);
+  if (!kb.bu) kb.bu = dalloc<float>(nb);
+  if (!kb.bv) kb.bv = dalloc<float>(nb);
+  if (!kb.sorted) kb.sorted = dalloc<double>(4 * (size_t)c->kln_npt * c->kln_nn);
+  float* tab = dalloc<float>(2 * kln_breaks_doubles(c->kln_npt, c->kln_nn));
+  kb.tab = tab;
+  const int rc = launch_kln_breaks(c->kln_nodes_d, c->kln_npt, c->kln_nn, kb, c->stream);
+  if (rc) {
+    kb.tab = nullptr;
+    (void)hipFree(tab);
+    check_launch(rc, "k_kln_breaks");
+  }
+}
+
 // MCnucl::setDensity for which_mc_model 1 (MCnucl.cpp:654-687): T_A, T_B
 // (MCnucl.cpp:398-478), then per-cell dN/dy from the table (reference) or
 // from the quadrature in every cell (kln_direct).  With the table on the
@@ -812,10 +832,11 @@ void run_kln_density(smc_ctx* c) {
     const int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)c->cap, ((size_t)1 << 28) / ncell_ev));
     const size_t cells = (size_t)chunk * ncell_ev;
     if (!c->kln_list) c->kln_list = dalloc<unsigned>(cells + 1);
+    ensure_kln_breaks(c);
     for (int e0 = 0; e0 < c->nev; e0 += chunk) {
       const size_t o = (size_t)e0 * ncell_ev, n = (size_t)std::min(chunk, c->nev - e0) * ncell_ev;
       check_launch(launch_kln_direct(a + o, b + o, s + o, n, c->kln_ptf, c->kln_nodes_f, c->kln_npt, c->kln_nn,
-                                     c->kln_kc, c->kln_list, c->kln_list + cells, c->stream),
+                                     c->kln_kc, c->kln_breaks, c->kln_list, c->kln_list + cells, c->stream),
                    "k_kln_direct");
     }
   } else {
@@ -1349,7 +1370,8 @@ void smc_destroy(smc_ctx* c) {
   void* ptrs[] = {c->buf.pos, c->buf.fluct, c->buf.wound, c->buf.pairs, c->buf.pfluct, c->buf.paw, c->buf.counts,
                   c->buf.bval, c->buf.raw, c->buf.src, c->buf.swin, c->dtab, c->grid, c->ta, c->tb, c->tmp, c->evout,
                   c->cm, c->band, c->mrects, c->nmrect, c->avg_rot, c->avg_acc, c->avg_sum, c->avg_part, c->avg_ext, c->aux0,
-                  c->aux1, c->grid64, c->spec_src, c->spec_swin, c->spec_counts, c->kln_table, c->kln_ptf, c->kln_nodes_f, c->kln_ptd, c->kln_nodes_d, c->kln_list};
+                  c->aux1, c->grid64, c->spec_src, c->spec_swin, c->spec_counts, c->kln_table, c->kln_ptf, c->kln_nodes_f, c->kln_ptd, c->kln_nodes_d, c->kln_list,
+                  c->kln_breaks.bu, c->kln_breaks.bv, c->kln_breaks.sorted, c->kln_breaks.tab};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   for (void* q : c->dif_alloc)

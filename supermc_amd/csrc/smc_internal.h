@@ -284,9 +284,21 @@ int launch_diff_moments(const DevCfg& cfg, const EvBufs& b, const DiffBufs& d, c
                         double ffdxdy, double* out, void* stream);
 int launch_diff_backward(const DevCfg& cfg, const EvBufs& b, const SmearSpec& spec, const DiffBufs& d, int nev,
                          const double* cot_dev, double ffdxdy, float* G, const double* theta, void* stream);
+// breakpoint tables of the per-cell quadrature (smc_kln_direct.hip): bu, bv
+// [npt][nn + 1] floats, sorted [npt][nn] double4 (build only), tab
+// kln_breaks_doubles() float2; all null: the node-by-node kernel
+struct KlnBreaks {
+  float* bu;
+  float* bv;
+  void* sorted;
+  void* tab;
+};
+bool kln_breaks_fit(int npt, int nn);
+size_t kln_breaks_doubles(int npt, int nn);
+int launch_kln_breaks(const void* nodes_d, int npt, int nn, const KlnBreaks& kb, void* stream);
 int launch_kln_direct(const float* ta, const float* tb, float* out, size_t ncell, const void* ptf,
-                      const void* nodes, int npt, int nn, const KlnConst& kc, unsigned* list, unsigned* count,
-                      void* stream);  // list: ncell entries, count: one (device scratch of the caller)
+                      const void* nodes, int npt, int nn, const KlnConst& kc, const KlnBreaks& kb, unsigned* list,
+                      unsigned* count, void* stream);  // list: ncell entries, count: one (device scratch of the caller)
 int launch_kln_points(const double* ta, const double* tb, double* out, int n, const void* ptd,
                       const void* nodes, int npt, int nn, const KlnConst& kc, void* stream);
 int launch_kln_table(const float* ta, const float* tb, float* out, int ncell_ev, int nev, int ny,

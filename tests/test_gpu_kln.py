@@ -150,6 +150,27 @@ def test_kln_direct_density_matches_fp64_quadrature():
             assert abs(s[1][ix, iy] - ref) <= 1e-5 * smax
 
 
+@pytest.mark.parametrize("nodes", [(1, 1, 2), (3, 5, 7), (5, 16, 2), (9, 31, 33), (2, 48, 63), (2, 49, 63)])
+def test_kln_direct_node_counts_match_fp64_quadrature(nodes):
+    """Node tables at the edges of the per-cell quadrature: fewer pT nodes
+    than the four waves that share them, one padded step of 16, odd counts,
+    and the two sides of the largest table that is interpolated (1536 nodes
+    per pT, then 1568).  The FP64 node sum on the same T_A, T_B is the
+    reference.  FP32 rounding: T_A g, its reciprocal, the interpolated or
+    summed terms and alpha_s are a few ulp each, below 1e-5 relative of the
+    largest cell."""
+    p = _kln_params(kln_direct=1, max_events=2, kln_n_pt=nodes[0], kln_n_kt=nodes[1], kln_n_phi=nodes[2])
+    xa, xb, bs = H.cpu_configs(p, 2, seed=12, bvals=np.array([3.0, 12.0]))
+    with _ctx(p) as ctx:
+        ctx.set_positions(xa, xb, bs)
+        s, _, _ = ctx.density()
+        ta, tb = ctx.thickness()
+        for e in range(2):
+            ref = ctx.kln_dndy(ta[e].ravel().astype(np.float64), tb[e].ravel().astype(np.float64))
+            assert ref.max() > 0
+            assert H.rel_linf(s[e].ravel(), ref) <= 1e-5
+
+
 def test_kln_table_overflow_sets_status():
     # tmax = 3 without subdivision: the table ends at T = 10/sigma, below the
     # centre of a central Pb+Pb event (MCnucl.cpp:665-670 stops the run)
