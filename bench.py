@@ -801,7 +801,7 @@ def main():
         # tile shape chosen on the warm-up batch (smc_autotune; grids do not depend on it)
         best, ms = ctx.autotune(reps=2)
         tune = dict(variant=best, ms_per_variant=[round(float(m), 3) for m in ms],
-                    variants=["32x64 chunk 8", "16x64 chunk 8", "32x64 chunk 4", "64x64 chunk 8", "64x32 rows interleaved"])
+                    variants=["by batch size", "1 wave per tile", "4 waves per tile", "16 waves per tile"])
     ctx.set_timing(True)
     t0 = time.perf_counter()
     for k in range(args.steps):

@@ -367,8 +367,8 @@ smc_status smc_set_systems(smc_ctx* ctx, int nsys, const smc_params* systems, in
 smc_status smc_get_event_system(smc_ctx* ctx, int ev, int* system);  /* -1: unmixed batch */
 
 /* Tile shapes of the exact-footprint smearing kernel (no counterpart in
- * the reference): 0 = 32 x 64 tiles, 8-row chunks (default); 1 = 16 x 64;
- * 2 = 32 x 64, 4-row chunks; 3 = 64 x 64.  Every shape gives the same grids.
+ * the reference): 32 x 64 tiles with one (1), four (2) or sixteen (3) waves
+ * each; 0 (default) chooses by the batch.  Every shape gives the same grids.
  * smc_autotune times each on the ctx's current events (reps launches after
  * a warm-up), keeps the fastest, and returns it with the per-shape times in
  * ms[SMC_TILE_VARIANTS] (either pointer may be NULL). */

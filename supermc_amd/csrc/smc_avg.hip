@@ -211,9 +211,10 @@ __global__ __launch_bounds__(256) void k_spectator_src(DevCfg cfg, EvBufs buf, E
   int4* swin = sb.swin + (size_t)e * sb.src_cap;
   if (t < 4) s_bb[t] = (t & 1) ? -1 : 0x7FFFFFFF;
   int bb[4] = {0x7FFFFFFF, -1, 0x7FFFFFFF, -1};
-  int base = 0;
+  int base = 0, nspec[2] = {0, 0};
   for (int nu = 0; nu < 2; ++nu) {
     const int A = cfg.nuc[nu].A;
+    nspec[nu] = -base;
     for (int i0 = 0; i0 < A; i0 += 256) {
       const int i = i0 + t;
       const bool spec = i < A && wound[nu * kAMax + i] == -1;  // -2: no nucleon in this slot
@@ -239,6 +240,7 @@ __global__ __launch_bounds__(256) void k_spectator_src(DevCfg cfg, EvBufs buf, E
       }
       base += s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     }
+    nspec[nu] += base;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -256,7 +258,9 @@ __global__ __launch_bounds__(256) void k_spectator_src(DevCfg cfg, EvBufs buf, E
   __syncthreads();
   if (t == 0) {
     int* c = sb.counts + (size_t)e * 8;
-    for (int q = 0; q < 5; ++q) c[q] = buf.counts[(size_t)e * 8 + q];
+    c[0] = nspec[0];  // the list's sources per kind
+    c[1] = nspec[1];
+    for (int q = 2; q < 5; ++q) c[q] = buf.counts[(size_t)e * 8 + q];
     c[5] = base;
     const bool none = s_bb[0] >= s_bb[1];
     c[6] = none ? 0 : (s_bb[0] | (s_bb[1] << 16));

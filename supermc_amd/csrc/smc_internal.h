@@ -110,6 +110,7 @@ struct EvBufs {
   int4* src;       // [ev][src_cap] {x_h, y_h, fluct bits, kind}
   int4* swin;      // [ev][src_cap] footprints {box x, box y, 5w x, 5w y}, lo | hi << 16
   int src_cap;
+  int* order;      // [ev] scratch of the smearing launches: the events, longest source lists first
 };
 
 // Event status bits
@@ -223,8 +224,7 @@ constexpr int kAccumSegments = 32;
 int launch_accum_avg(const float* grid, const int* counts, int nx, int ny, int nev, const unsigned char* accept,
                      double ff, double* part, double* sum, void* stream, const float* grid2 = nullptr);
 constexpr int kTileVariants = 4;
-int tile_units(const DevCfg& cfg);  // smearing tiles per event of cfg's variant (units of SmearSpec::cm_out)
-int tile_units_max(const DevCfg& cfg);  // the most over all variants (buffer sizing)
+int tile_units(const DevCfg& cfg);  // 32 x 64 smearing tiles per event (units of SmearSpec::cm_out)
 // exact-footprint smearing as an MFMA contraction (smc_mtile.hip): prec 0
 // FP32, 1 BF16x3, 2 BF16x6; ktab (tmax x tmax) selects the fused MC-KLN
 // epilogue.  Its centre-of-mass partials have mtile_units(cfg) units (the
@@ -270,7 +270,7 @@ int launch_p3d_smear(const P3dCfg& c, int nev, const double* src, const int* src
 double regge_sigma_inel(double ecm);
 
 // MC-KLN density in one pass: T_A (acc 0) and T_B (acc 1) of s, then dN/dy
-// from the tmax x tmax table at (T_A/dT, T_B/dT), in the ctx's tile shape;
+// from the tmax x tmax table at (T_A/dT, T_B/dT);
 // s.cm_out gets the output's centre-of-mass partials (tile_units per event)
 // when set
 int launch_tile_kln(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev, float* out,

@@ -19,25 +19,58 @@
 // exact disk.  Without a cut (cut2 = 1e30) K = 2^64, nothing flushes and
 // the footprint is the integer window alone.
 //
-// One wavefront owns a tile of TR rows x 64 columns in TR accumulators per
-// lane (lane = column).  It selects the sources whose window meets the tile
-// in source order (ballot compaction, so the summation order is fixed).
-// Row factors K gx(row) go through LDS (broadcast float4 reads); with PAIR
-// the two half-waves compute them for two sources at once.  Every lane
-// computes gy(column) itself, and chunks of CH rows that a source's window
-// misses are skipped by a uniform branch.  The launch uses TR = 32, CH = 8,
-// PAIR (measured against TR 16/64, CH 4/16/32, unpaired, and a 32-column
-// layout with interleaved half-wave rows).
+// One workgroup owns a tile of 32 rows x 64 columns of an event: one wave, or
+// four or sixteen where a batch has too few tiles to fill the chip (a tile is
+// a serial chain over its sources).  The sources of the list whose window
+// meets the tile are selected in source order (ballot compaction, so every
+// cell adds its terms in one fixed order whatever the shape) and taken a few
+// at a time: row factors K gx and column factors gy go to LDS once per source,
+// then each lane adds its cells.
+//
+// In the one-wave kernel lane (q, c) = (lane / 16, lane % 16) holds the cells of rows q + 4 i and
+// columns c + 16 k: a source costs a lane TR / 4 row and 4 column factors, read
+// as float4, for TR cells.  (With lane = column a cell needs its own row
+// factor from LDS, and the LDS return path, 128 B per clock and CU, is as busy
+// as the VALU: a layout with fewer VALU instructions then gained nothing.)
+// Register (i, k) of a wave is a 4 x 16 patch, so a source's work is skipped in
+// units of 16 x 16 cells that its window or its disk does not reach: 3,800 cell
+// slots of 6,700 in 8-row chunks of 64 columns remain for a 51-cell window.  At the end the 4 x 4 blocks (q, k) are
+// transposed across the lane groups, and a lane holds one column again:
+// stores of 64 consecutive cells.
 #include "smc_device.h"
 
 namespace smc {
 
-struct TileEntry {
-  int xh, yh;
+// a selected source: position (half-quanta) and window per axis, weight, and
+// the units of the wave's tile that it reaches (bit 4 row unit + column block)
+struct alignas(8) TileEntry {
+  int xh, xw;
+  int yh, yw;
   float w;
-  int xw, yw;
-  int pad;
+  unsigned units;
 };
+
+constexpr int kTileRows = 32;  // rows of a workgroup's tile
+
+// The 4 x 4 transpose of v over (lane group of 16, register):
+// v[k] of group q <- v[q] of group k.
+__device__ __forceinline__ void transpose_groups(float (&v)[4]) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const auto swap32 = [](float& a, float& b) {
+    const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r.x);
+    b = __uint_as_float(r.y);
+  };
+  const auto swap16 = [](float& a, float& b) {
+    const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r.x);
+    b = __uint_as_float(r.y);
+  };
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+  swap16(v[0], v[1]);
+  swap16(v[2], v[3]);
+}
 
 // The MC-KLN density of MCnucl::setDensity (which_mc_model 1,
 // MCnucl.cpp:654-687) fused into the smearing: T_A and T_B accumulate in two
@@ -73,245 +106,684 @@ __device__ __forceinline__ float kln_cell(float A, float B, const KlnTab& kt, bo
   return (float)(axx * x * x + axy * x * y + ayy * y * y + bx * x + by * y + v00);
 }
 
+// Event and tile of a workgroup.  Workgroups go to the 8 XCDs round-robin by
+// linear id; this mapping gives all tiles of an event one XCD (one L2 holds
+// its source list, and the partial cache lines at tile edges meet in that
+// L2).  spread: the tiles of an event go to all XCDs instead (few events: one
+// XCD has 32 CUs).
+struct TileAt {
+  int e, tile, T, R0, c0;  // e < 0: no event
+  bool col_live;  // the event's source rectangle reaches the tile's columns
+  int x0, x1;     // its rows
+};
+__device__ __forceinline__ TileAt tile_at(const DevCfg& cfg, const EvBufs& buf, int nev, int spread,
+                                          const int* order) {
+  const int ntx = (cfg.nx + kTileRows - 1) / kTileRows;
+  TileAt at;
+  at.T = ntx * ((cfg.ny + 63) >> 6);
+  const unsigned L = blockIdx.x, rg = L % (8u * at.T);
+  at.e = spread ? (int)(L / at.T) : (int)(8u * (L / (8u * at.T)) + rg % 8u);
+  at.tile = spread ? (int)(L % at.T) : (int)(rg / 8u);
+  at.R0 = kTileRows * (at.tile % ntx);
+  at.c0 = 64 * (at.tile / ntx);
+  at.e = at.e < nev ? (order ? order[at.e] : at.e) : -1;
+  const int e = max(at.e, 0);
+  const int rx = buf.counts[(size_t)e * 8 + 6], ry = buf.counts[(size_t)e * 8 + 7];
+  at.col_live = (ry & 0xffff) < at.c0 + 64 && (ry >> 16) > at.c0;
+  at.x0 = rx & 0xffff;
+  at.x1 = rx >> 16;
+  return at;
+}
+
+// The range of event e's source list that holds accumulator want's sources
+// (the list is the projectile's participants, the target's, then the pairs).
+__device__ __forceinline__ int2 source_range(const EvBufs& buf, const SmearSpec& spec, int e, int want) {
+  const int* cnt = buf.counts + (size_t)e * 8;
+  const int K = cnt[5];
+  const int end[3] = {min(cnt[0], K), min(cnt[0] + cnt[1], K), K};
+  int2 r = make_int2(K, 0);
+#pragma unroll
+  for (int kind = 0; kind < 3; ++kind)
+    if (spec.enabled[kind] && spec.acc[kind] == want) {
+      r.x = min(r.x, kind ? end[kind - 1] : 0);
+      r.y = end[kind];
+    }
+  return r;
+}
+
+// The source (s, wv4) as an entry, with units != 0 if it belongs to
+// accumulator want and reaches the rows r0 .. r0 + UROWS NU - 1 and columns
+// c0 .. c0 + 63: bit 4 u + kb for rows [r0 + UROWS u, + UROWS), columns
+// [c0 + 16 kb, + 16).  A unit is reached if the window meets it and its
+// nearest cell lies within reach2: cut2 and a margin that covers the float
+// product's own boundary (a few ulp of exp(-cut2 / 2w^2)).
+template <int UROWS, int NU>
+__device__ __forceinline__ TileEntry tile_entry(const DevCfg& cfg, const SmearSpec& spec, const int4& s,
+                                                const int4& wv4, int want, int r0, int c0) {
+  TileEntry en{0, 0, 0, 0, 0.f, 0u};
+  const int kind = s.w;
+  if (!(spec.enabled[kind] && spec.acc[kind] == want)) return en;
+  en.xh = s.x;
+  en.yh = s.y;
+  en.xw = (spec.win[kind] == kWinBox) ? wv4.x : wv4.z;
+  en.yw = (spec.win[kind] == kWinBox) ? wv4.y : wv4.w;
+  en.w = spec.scale[kind] * (spec.use_fluct[kind] ? __int_as_float(s.z) : 1.f) * cfg.tile_w;
+  const int xlo = en.xw & 0xffff, xhi = en.xw >> 16, ylo = en.yw & 0xffff, yhi = en.yw >> 16;
+  if (!(xlo < r0 + UROWS * NU && xhi > r0 && ylo < c0 + 64 && yhi > c0)) return en;
+  const float reach2 = cfg.cut2 * 1.001f;
+  const float sx = (float)(en.xh * kH - cfg.xmin), sy = (float)(en.yh * kH - cfg.ymin);
+  const float fdx = (float)cfg.dx, fdy = (float)cfg.dy;
+  float d2y[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    const int a = max(c0 + 16 * kb, ylo), b = min(c0 + 16 * kb + 16, yhi) - 1;
+    const float d = fmaxf(0.f, fmaxf(a * fdy - sy, sy - b * fdy));
+    d2y[kb] = a <= b ? d * d : 3.0e38f;
+  }
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int a = max(r0 + UROWS * u, xlo), b = min(r0 + UROWS * (u + 1), xhi) - 1;
+    const float d = fmaxf(0.f, fmaxf(a * fdx - sx, sx - b * fdx));
+    if (a > b) continue;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+      if (d * d + d2y[kb] <= reach2) en.units |= 1u << (4 * u + kb);
+  }
+  return en;
+}
+
 // EPI 1 (MC-KLN) and 2 (sqrt(T_A T_B), MCnucl.cpp:762-811): the sources of
 // accumulator 0 (T_A), then those of accumulator 1 (T_B), each set in source
 // order, and the output is the cell's dN/dy from the table, or
 // sqrtf(T_A T_B) of the stored floats.  EPI 0: the sources of accumulator
 // acc_sel only.
-template <int TR, int CH, bool PAIR, int EPI>
-__global__ __launch_bounds__(64) void k_tile(DevCfg cfg, EvBufs buf, SmearSpec spec, int acc_sel, int nev, float* out,
-                                             KlnTab kt) {
-  static_assert(TR % CH == 0 && CH % 4 == 0 && TR <= 64 && (!PAIR || TR <= 32), "tile rows");
-  __shared__ TileEntry wl[64];
-  __shared__ float4 rd[2][TR / 4];  // K gx(row) of the current source(s), 0 outside the window
-  const int lane = threadIdx.x;
-  const int nx = cfg.nx, ny = cfg.ny;
-  const int ntx = (nx + TR - 1) / TR;
-  // Workgroups go to the 8 XCDs round-robin by linear id; this mapping
-  // gives all tiles of an event one XCD (one L2 holds its source list, and
-  // the partial cache lines at tile edges meet in that L2).
-  const int T = ntx * ((ny + 63) >> 6);
-  const unsigned L = blockIdx.x, rg = L % (8u * T);
-  const int e = (int)(8u * (L / (8u * T)) + rg % 8u), tile = (int)(rg / 8u);
-  if (e >= nev) return;
-  const int r0 = TR * (tile % ntx), c0 = 64 * (tile / ntx);
-  // exp2 argument -(d_h)^2 kH^2 inv2w2 log2 e with d_h in half-quanta (kH^2 is a power of two)
-  const float cq = cfg.inv2w2 * 1.4426950408889634f * (kHf * kHf);
-  const float kk = cfg.tile_k;
-  const int col = c0 + lane;
-  const int ygh = (int)llrint((cfg.ymin + col * cfg.dy) / kH);
-  const int rl = PAIR ? (lane & 31) : lane;     // row this lane computes a factor for
-  const int rs = PAIR ? (lane >> 5) : 0;        // which of the pair
-  const int myrow = r0 + (rl < TR ? rl : 0);
-  const int rowh = (int)llrint((cfg.xmin + myrow * cfg.dx) / kH);
-  const int K = buf.counts[(size_t)e * 8 + 5];
-  const int4* src = buf.src + (size_t)e * buf.src_cap;
-  const int4* swin = buf.swin + (size_t)e * buf.src_cap;
-  float* rdf = reinterpret_cast<float*>(&rd[0][0]);
-
+//
+// What the kernels below do with the sums of rows r0 .. r0 + TR - 1 (lane =
+// column; aA: T_A where there are two): the epilogue, the stores, and per
+// column the sums p of each 8 rows for the centre-of-mass partials.
+template <int TR, int EPI>
+__device__ __forceinline__ void tile_finish(const DevCfg& cfg, const EvBufs& buf, const TileAt& at, int r0, bool live,
+                                            float (&a)[TR], const float (&aA)[EPI ? TR : 1], const KlnTab& kt,
+                                            float* out, double (&p)[TR / 8][2]) {
   constexpr bool TWO = EPI != 0;
-  float acc[TR], accA[TWO ? TR : 1];  // accA: T_A while the second pass fills acc with T_B
-#pragma unroll
-  for (int r = 0; r < TR; ++r) acc[r] = 0.f;
-  // tiles outside the event's source rectangle stay zero
-  const int rx = buf.counts[(size_t)e * 8 + 6], ry = buf.counts[(size_t)e * 8 + 7];
-  const bool live = (rx & 0xffff) < r0 + TR && (rx >> 16) > r0 && (ry & 0xffff) < c0 + 64 && (ry >> 16) > c0;
-  if (!live && spec.sparse) {  // nothing to store: zero centre-of-mass partials only
-    if (spec.cm_out && lane < 4) spec.cm_out[((size_t)e * T + tile) * 4 + lane] = 0.0;
-    return;
-  }
-
-  auto fma_phase = [&](const float4* rr, float gy, float wq, int xw) {
-    const int xlo = xw & 0xffff, xhi = xw >> 16;
-#pragma unroll
-    for (int c = 0; c < TR / CH; ++c) {
-      // chunks of CH rows that the source's window misses are skipped
-      if (CH == TR || (r0 + CH * c < xhi && r0 + CH * c + CH > xlo)) {
-#pragma unroll
-        for (int i = c * CH / 4; i < (c + 1) * CH / 4; ++i) {
-          const float4 v = rr[i];
-          acc[4 * i] = fmaf(v.x * gy, wq, acc[4 * i]);
-          acc[4 * i + 1] = fmaf(v.y * gy, wq, acc[4 * i + 1]);
-          acc[4 * i + 2] = fmaf(v.z * gy, wq, acc[4 * i + 2]);
-          acc[4 * i + 3] = fmaf(v.w * gy, wq, acc[4 * i + 3]);
-        }
-      }
-    }
-  };
-  auto col_factor = [&](const TileEntry& q) {
-    const int ylo = q.yw & 0xffff, yhi = q.yw >> 16;
-    const float dy = (float)(ygh - q.yh);
-    return (col >= ylo && col < yhi) ? __builtin_amdgcn_exp2f(-(dy * dy) * cq) : 0.f;
-  };
-
-  for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
-   if (TWO && pass == 1) {
-#pragma unroll
-    for (int r = 0; r < TR; ++r) {
-      accA[TWO ? r : 0] = acc[r];
-      acc[r] = 0.f;
-    }
-   }
-   const int want = TWO ? pass : acc_sel;
-   for (int sub = 0; live && sub < K; sub += 64) {
-    const int k = sub + lane;
-    bool sel = false;
-    TileEntry en{0, 0, 0.f, 0, 0, 0};
-    if (k < K) {
-      const int4 s = src[k];
-      const int kind = s.w;
-      if (spec.enabled[kind] && spec.acc[kind] == want) {
-        const int4 wv = swin[k];
-        en.xh = s.x;
-        en.yh = s.y;
-        en.xw = (spec.win[kind] == kWinBox) ? wv.x : wv.z;
-        en.yw = (spec.win[kind] == kWinBox) ? wv.y : wv.w;
-        en.w = spec.scale[kind] * (spec.use_fluct[kind] ? __int_as_float(s.z) : 1.f) * cfg.tile_w;
-        const int xlo = en.xw & 0xffff, xhi = en.xw >> 16, ylo = en.yw & 0xffff, yhi = en.yw >> 16;
-        sel = xlo < r0 + TR && xhi > r0 && ylo < c0 + 64 && yhi > c0;
-      }
-    }
-    const unsigned long long m = __ballot(sel);
-    if (sel) wl[__popcll(m & ((1ull << lane) - 1ull))] = en;
-    const int n = __popcll(m);
-    __builtin_amdgcn_wave_barrier();
-    for (int g = 0; g < n; g += (PAIR ? 2 : 1)) {
-      // row factors: lanes rl < TR of half rs for source g + rs
-      {
-        const int gi = (PAIR && g + rs < n) ? g + rs : g;
-        const TileEntry q = wl[gi];
-        if (rl < TR) {
-          const float dx = (float)(rowh - q.xh);
-          const int xlo = q.xw & 0xffff, xhi = q.xw >> 16;
-          const float gx = kk * __builtin_amdgcn_exp2f(-(dx * dx) * cq);
-          rdf[rs * TR + rl] = (myrow >= xlo && myrow < xhi) ? gx : 0.f;
-        }
-      }
-      const TileEntry q0 = wl[g];
-      const float gy0 = col_factor(q0);
-      const int xw0 = __builtin_amdgcn_readfirstlane(q0.xw);
-      __builtin_amdgcn_wave_barrier();
-      fma_phase(rd[0], gy0, q0.w, xw0);
-      if constexpr (PAIR) {
-        if (g + 1 < n) {
-          const TileEntry q1 = wl[g + 1];
-          const float gy1 = col_factor(q1);
-          const int xw1 = __builtin_amdgcn_readfirstlane(q1.xw);
-          fma_phase(rd[1], gy1, q1.w, xw1);
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-    __builtin_amdgcn_wave_barrier();
-   }
-  }
+  const int lane = threadIdx.x & 63, col = at.c0 + lane, nx = cfg.nx, ny = cfg.ny;
   const float so = cfg.tile_out;
   if constexpr (EPI == 2) {
     // sqrt(T_A T_B) of the stored floats; the product is formed in double,
     // so the result does not depend on the f32 denormal mode of this file
 #pragma unroll
-    for (int r = 0; r < TR; ++r) acc[r] = (float)sqrt((double)(accA[r] * so) * (double)(acc[r] * so));
+    for (int r = 0; r < TR; ++r) a[r] = (float)sqrt((double)(aA[r] * so) * (double)(a[r] * so));
   }
-  if constexpr (EPI == 1) {  // dN/dy from (T_A, T_B) = (accA, acc) as stored floats
+  if constexpr (EPI == 1) {  // dN/dy from (T_A, T_B) = (aA, a) as stored floats
     bool off = false;
 #pragma unroll
     for (int r = 0; r < TR; ++r)
-      acc[r] = (live && col < ny && r0 + r < nx) ? kln_cell(accA[r] * so, acc[r] * so, kt, off) : 0.f;
-    if (off) atomicOr(&buf.counts[(size_t)e * 8 + 3], kStKlnTable);
+      a[r] = (live && col < ny && r0 + r < nx) ? kln_cell(aA[r] * so, a[r] * so, kt, off) : 0.f;
+    if (off) atomicOr(&buf.counts[(size_t)at.e * 8 + 3], kStKlnTable);
   }
-  const float os = TWO ? 1.f : so;  // stored value = acc * os
-  if (spec.cm_out) {  // centre-of-mass partials of the stored grid values
-    double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-    for (int r = 0; r < TR; ++r) {
-      if (col < ny && r0 + r < nx) {
-        const double v = (double)(acc[r] * os);
-        s0 += v;
-        s1 = fma(cfg.xmin + (r0 + r) * cfg.dx, v, s1);
-      }
-    }
-    double s2 = (col < ny) ? (cfg.ymin + col * cfg.dy) * s0 : 0.0;
-    s0 = wave_sum(s0);
-    s1 = wave_sum(s1);
-    s2 = wave_sum(s2);
-    if (lane == 0) {
-      double* p = spec.cm_out + ((size_t)e * T + tile) * 4;
-      p[0] = s0;
-      p[1] = s1;
-      p[2] = s2;
-      p[3] = 0.0;
-    }
-  }
-  if (col >= ny) return;
+  const float os = TWO ? 1.f : so;  // stored value = a * os
   const size_t N = (size_t)nx * ny;
+  float* o = out + (size_t)at.e * N + (size_t)r0 * ny + col;
 #pragma unroll
   for (int r = 0; r < TR; ++r) {
-    const int ix = r0 + r;
-    if (ix < nx) out[(size_t)e * N + (size_t)ix * ny + col] = acc[r] * os;
+    if (r % 8 == 0) p[r / 8][0] = p[r / 8][1] = 0.0;
+    if (col < ny && r0 + r < nx) {
+      const float f = a[r] * os;
+      o[(size_t)r * ny] = f;
+      const double v = (double)f;
+      p[r / 8][0] += v;
+      p[r / 8][1] = fma(cfg.xmin + (r0 + r) * cfg.dx, v, p[r / 8][1]);
+    }
   }
 }
 
-constexpr int kTileRows = 32;
-
-// Tile shapes the autotuner chooses from (rows x 64 columns, row chunk,
-// paired row factors).  Every shape adds the same products in the same
-// source order per cell, so the grids do not depend on the choice.
-//   0: 32 rows, chunks of 8, paired   (the default)
-//   1: 16 rows, chunks of 8, paired
-//   2: 32 rows, chunks of 4, paired
-//   3: 64 rows, chunks of 8, unpaired
-constexpr int kVariantRows[kTileVariants] = {32, 16, 32, 64};
-
-static int units_for_rows(const DevCfg& cfg, int rows) { return ((cfg.nx + rows - 1) / rows) * ((cfg.ny + 63) / 64); }
-static int variant_of(const DevCfg& cfg) {
-  return (cfg.tile_variant >= 0 && cfg.tile_variant < kTileVariants) ? cfg.tile_variant : 0;
-}
-int tile_units(const DevCfg& cfg) { return units_for_rows(cfg, kVariantRows[variant_of(cfg)]); }
-int tile_units_max(const DevCfg& cfg) {
-  int m = 0;
-  for (int v = 0; v < kTileVariants; ++v) m = max(m, units_for_rows(cfg, kVariantRows[v]));
-  return m;
+// A tile's centre-of-mass partials from its column sums s0 = sum v, s1 = sum x v
+__device__ __forceinline__ void tile_cm(const DevCfg& cfg, const TileAt& at, double s0, double s1, double* cm_out) {
+  const int lane = threadIdx.x & 63, col = at.c0 + lane;
+  double s2 = (col < cfg.ny) ? (cfg.ymin + col * cfg.dy) * s0 : 0.0;
+  s0 = wave_sum(s0);
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  if (lane == 0) {
+    double* p = cm_out + ((size_t)at.e * at.T + at.tile) * 4;
+    p[0] = s0;
+    p[1] = s1;
+    p[2] = s2;
+    p[3] = 0.0;
+  }
 }
 
-template <int TR, int CH, bool PAIR>
-static void launch_tr(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev, float* out0, float* out1,
-                      hipStream_t st) {
-  // one dimension: tiles x events padded to a multiple of the 8 XCDs
-  const dim3 grid((unsigned)(((cfg.nx + TR - 1) / TR) * ((cfg.ny + 63) / 64)) * (unsigned)((nev + 7) / 8 * 8));
-  const KlnTab none{nullptr, 0, 1.0};
-  if (s.combine == 1) {  // sqrt(T_A T_B) in one launch, with the partials of the combined grid
-    hipLaunchKernelGGL((k_tile<TR, CH, PAIR, 2>), grid, dim3(64), 0, st, cfg, b, s, 0, nev, out0, none);
+// ---- one wave per tile, for batches that fill the chip: VALU issue bound (two
+// instructions per cell slot, about 60 per source and tile around them).
+// 4 sources' factors in LDS at a time and 72 VGPRs (7 waves per SIMD): 8.93 ms
+// per 50,000 Pb+Pb events of 261^2 cells; 8 sources 9.45 (7 waves) and 9.41
+// (74 VGPRs, 6 waves), 8 waves with 4 sources 9.2.  One column per lane with
+// row factors broadcast from LDS took 11.0.  The two-accumulator forms keep
+// their 106 VGPRs: spilling them cost a quarter.
+constexpr int kSB = 4;
+
+template <int EPI>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EPI ? 1 : 7, EPI ? 8 : 7))) void k_tile(DevCfg cfg, EvBufs buf, SmearSpec spec, int acc_sel, int nev, int spread,
+                                             const int* order, float* out, KlnTab kt) {
+  constexpr int TR = kTileRows, NI = TR / 4;
+  constexpr int UR = 4, NU = NI / UR;  // row groups per unit, row units
+  constexpr bool TWO = EPI != 0;
+  __shared__ TileEntry wl[128];
+  __shared__ float4 fx_s[kSB][TR / 4];  // K gx: row q + 4 i at q NI + i
+  __shared__ float4 fy_s[kSB][16];      // gy: column c + 16 k at 4 c + k
+  const int lane = threadIdx.x, q = lane >> 4, c = lane & 15;
+  const TileAt at = tile_at(cfg, buf, nev, spread, order);
+  if (at.e < 0) return;
+  const int e = at.e, r0 = at.R0, c0 = at.c0;
+  // tiles outside the event's source rectangle stay zero
+  const bool live = at.col_live && at.x0 < r0 + TR && at.x1 > r0;
+  if (!live && spec.sparse) {  // nothing to store: zero centre-of-mass partials only
+    if (spec.cm_out && lane < 4) spec.cm_out[((size_t)e * at.T + at.tile) * 4 + lane] = 0.0;
     return;
   }
-  SmearSpec s1 = s;  // partials only for a single accumulator
-  if (s.combine != 0) s1.cm_out = nullptr;
-  hipLaunchKernelGGL((k_tile<TR, CH, PAIR, 0>), grid, dim3(64), 0, st, cfg, b, s1, 0, nev, out0, none);
-  if (s.combine != 0)
-    hipLaunchKernelGGL((k_tile<TR, CH, PAIR, 0>), grid, dim3(64), 0, st, cfg, b, s1, 1, nev, out1, none);
+  // exp2 argument -(d_h)^2 kH^2 inv2w2 log2 e with d_h in half-quanta (kH^2 is a power of two)
+  const float cq = cfg.inv2w2 * 1.4426950408889634f * (kHf * kHf);
+  const float kk = cfg.tile_k;
+  const int col = c0 + lane;
+  const int ygh = (int)llrint((cfg.ymin + col * cfg.dy) / kH);
+  const int rl = lane & (TR - 1), rs = lane / TR;  // row and source of a pass whose factor this lane computes
+  const int rowh = (int)llrint((cfg.xmin + (r0 + rl) * cfg.dx) / kH);
+  const int4* src = buf.src + (size_t)e * buf.src_cap;
+  const int4* swin = buf.swin + (size_t)e * buf.src_cap;
+
+  float acc[NI][4], accA[TWO ? NI : 1][4];  // accA: T_A while the second pass fills acc with T_B
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[i][k] = 0.f;
+
+  for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
+    if (TWO && pass == 1) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          accA[TWO ? i : 0][k] = acc[i][k];
+          acc[i][k] = 0.f;
+        }
+    }
+    const int want = TWO ? pass : acc_sel;
+    const int2 kr = source_range(buf, spec, e, want);
+    const int K = live ? kr.y : 0;
+    int n = 0;  // selected sources waiting in wl
+    for (int sub = kr.x; sub < K || n > 0;) {
+      // select until 64 wait or the list ends
+      while (sub < K && n < 64) {
+        const int k = sub + lane;
+        sub += 64;
+        TileEntry en{0, 0, 0, 0, 0.f, 0u};
+        if (k < K) en = tile_entry<4 * UR, NU>(cfg, spec, src[k], swin[k], want, r0, c0);
+        const unsigned long long m = __ballot(en.units != 0u);
+        if (en.units) wl[n + __popcll(m & ((1ull << lane) - 1ull))] = en;
+        n += __popcll(m);
+      }
+      __builtin_amdgcn_wave_barrier();
+      const int take = min(n, 64);
+      const TileEntry me = wl[lane];
+      for (int g = 0; g < take; g += kSB) {
+        const int ng = min(kSB, take - g);
+#pragma unroll
+        for (int p = 0; p < kSB; p += 64 / TR) {
+          if (p >= ng) break;
+          const int2 ex = *reinterpret_cast<const int2*>(&wl[g + p + rs].xh);
+          const float dx = (float)(rowh - ex.x);
+          const int xlo = ex.y & 0xffff, xhi = ex.y >> 16;
+          const float gx = kk * __builtin_amdgcn_exp2f(-(dx * dx) * cq);
+          reinterpret_cast<float*>(fx_s[p + rs])[(rl & 3) * NI + (rl >> 2)] =
+              (r0 + rl >= xlo && r0 + rl < xhi) ? gx : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < kSB; ++u) {
+          if (u >= ng) break;
+          const int yh = __builtin_amdgcn_readlane(me.yh, g + u), yw = __builtin_amdgcn_readlane(me.yw, g + u);
+          const int ylo = yw & 0xffff, yhi = yw >> 16;
+          const float dy = (float)(ygh - yh);
+          reinterpret_cast<float*>(fy_s[u])[4 * c + q] =
+              (col >= ylo && col < yhi) ? __builtin_amdgcn_exp2f(-(dy * dy) * cq) : 0.f;
+        }
+        __builtin_amdgcn_wave_barrier();
+        for (int u = 0; u < ng; ++u) {
+          const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(me.w), g + u));
+          const unsigned um = __builtin_amdgcn_readlane(me.units, g + u);
+          float x[NI];
+          const float* fx = reinterpret_cast<const float*>(fx_s[u]) + q * NI;
+#pragma unroll
+          for (int i = 0; i < NI; ++i) x[i] = fx[i];
+          const float4 y4 = fy_s[u][c];
+          const float y[4] = {y4.x, y4.y, y4.z, y4.w};
+#pragma unroll
+          for (int b = 0; b < 4 * NU; ++b) {
+            if ((um >> b) & 1u) {
+#pragma unroll
+              for (int i = (b >> 2) * UR; i < ((b >> 2) + 1) * UR; ++i)
+                acc[i][b & 3] = fmaf(x[i] * y[b & 3], w, acc[i][b & 3]);
+            }
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+      n -= take;
+      if (lane < n) wl[lane] = wl[64 + lane];  // n <= 63 are left
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  // lane = column again: a[4 i + j] is row 4 i + j
+  float a[TR], aA[TWO ? TR : 1];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    transpose_groups(acc[i]);
+    if constexpr (TWO) transpose_groups(accA[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[4 * i + j] = acc[i][j];
+      if constexpr (TWO) aA[4 * i + j] = accA[i][j];
+    }
+  }
+  double p[TR / 8][2];
+  tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out, p);
+  if (spec.cm_out) {
+    double s0 = p[0][0], s1 = p[0][1];
+#pragma unroll
+    for (int h = 1; h < TR / 8; ++h) {
+      s0 += p[h][0];
+      s1 += p[h][1];
+    }
+    tile_cm(cfg, at, s0, s1, spec.cm_out);
+  }
 }
 
-template <int TR, int CH, bool PAIR>
-static void launch_tr_kln(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev, float* out,
-                          const KlnTab& kt, hipStream_t st) {
-  const dim3 grid((unsigned)(((cfg.nx + TR - 1) / TR) * ((cfg.ny + 63) / 64)) * (unsigned)((nev + 7) / 8 * 8));
-  hipLaunchKernelGGL((k_tile<TR, CH, PAIR, 1>), grid, dim3(64), 0, st, cfg, b, s, 0, nev, out, kt);
+// ---- four waves of 8 rows per tile, between the two: the workgroup selects
+// 256 sources at a time and shares the factors of kGB4 sources, double-
+// buffered, one barrier per kGB4 sources.
+constexpr int kGB4 = 16;
+
+template <int EPI>
+__global__ __launch_bounds__(256) void k_tile4(DevCfg cfg, EvBufs buf, SmearSpec spec, int acc_sel, int nev, int spread,
+                                               const int* order, float* out, KlnTab kt) {
+  constexpr int NW = 4, TR = kTileRows / NW, NI = TR / 4;
+  constexpr bool TWO = EPI != 0;
+  __shared__ TileEntry wl[256];
+  __shared__ float fx_s[2][kGB4][kTileRows];  // K gx: row 8 v + q + 4 i at 8 v + 2 q + i
+  __shared__ float4 fy_s[2][kGB4][16];        // gy: column c + 16 k at 4 c + k
+  __shared__ int cnt_s[NW];
+  __shared__ double cm_s[NW][2][64];
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), q = lane >> 4, c = lane & 15;
+  const TileAt at = tile_at(cfg, buf, nev, spread, order);
+  if (at.e < 0) return;
+  const int e = at.e, R0 = at.R0, r0 = R0 + TR * wv, c0 = at.c0;
+  const bool live = at.col_live && at.x0 < R0 + kTileRows && at.x1 > R0;
+  if (!live && spec.sparse) {  // uniform over the workgroup
+    if (spec.cm_out && t < 4) spec.cm_out[((size_t)e * at.T + at.tile) * 4 + t] = 0.0;
+    return;
+  }
+  const float cq = cfg.inv2w2 * 1.4426950408889634f * (kHf * kHf);
+  const float kk = cfg.tile_k;
+  const int col = c0 + lane, row = R0 + (t & 31);  // of the factors this thread computes
+  const int ygh = (int)llrint((cfg.ymin + col * cfg.dy) / kH);
+  const int rowh = (int)llrint((cfg.xmin + row * cfg.dx) / kH);
+  const int fxi = (t & 24) + 2 * (t & 3) + ((t >> 2) & 1);
+  const int4* src = buf.src + (size_t)e * buf.src_cap;
+  const int4* swin = buf.swin + (size_t)e * buf.src_cap;
+
+  float acc[NI][4], accA[TWO ? NI : 1][4];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[i][k] = 0.f;
+
+  for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
+    if (TWO && pass == 1) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          accA[TWO ? i : 0][k] = acc[i][k];
+          acc[i][k] = 0.f;
+        }
+    }
+    const int want = TWO ? pass : acc_sel;
+    const int2 kr = source_range(buf, spec, e, want);
+    const int k0 = kr.x, K = live ? kr.y : 0;
+    int4 ps = make_int4(0, 0, 0, 0), pw = ps;  // this thread's source of the next 256
+    if (k0 + t < K) {
+      ps = src[k0 + t];
+      pw = swin[k0 + t];
+    }
+    for (int sub = k0; sub < K; sub += 256) {
+      TileEntry en{0, 0, 0, 0, 0.f, 0u};
+      if (sub + t < K) en = tile_entry<TR, NW>(cfg, spec, ps, pw, want, R0, c0);
+      if (sub + 256 + t < K) {
+        ps = src[sub + 256 + t];
+        pw = swin[sub + 256 + t];
+      }
+      const unsigned long long m = __ballot(en.units != 0u);
+      __syncthreads();  // the entries and counts of the last round are read
+      if (lane == 0) cnt_s[wv] = __popcll(m);
+      __syncthreads();
+      int n = 0, at_n = 0;
+#pragma unroll
+      for (int v = 0; v < NW; ++v) {
+        if (v == wv) at_n = n;
+        n += cnt_s[v];
+      }
+      if (en.units) wl[at_n + __popcll(m & ((1ull << lane) - 1ull))] = en;
+      __syncthreads();
+      for (int g = 0; g < n; g += kGB4) {
+        const int b = (g / kGB4) & 1, ng = min(kGB4, n - g);
+        // factors: rows of 8 sources, then columns of 4 sources, per pass
+#pragma unroll
+        for (int p = 0; p < kGB4; p += 8) {
+          const int s = p + (t >> 5);
+          if (s < ng) {
+            const int2 ex = *reinterpret_cast<const int2*>(&wl[g + s].xh);
+            const float dx = (float)(rowh - ex.x);
+            const int xlo = ex.y & 0xffff, xhi = ex.y >> 16;
+            const float gx = kk * __builtin_amdgcn_exp2f(-(dx * dx) * cq);
+            fx_s[b][s][fxi] = (row >= xlo && row < xhi) ? gx : 0.f;
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < kGB4; p += NW) {
+          const int s = p + wv;
+          if (s < ng) {
+            const int2 ey = *reinterpret_cast<const int2*>(&wl[g + s].yh);
+            const float dy = (float)(ygh - ey.x);
+            const int ylo = ey.y & 0xffff, yhi = ey.y >> 16;
+            reinterpret_cast<float*>(fy_s[b][s])[4 * c + q] =
+                (col >= ylo && col < yhi) ? __builtin_amdgcn_exp2f(-(dy * dy) * cq) : 0.f;
+          }
+        }
+        // the batch's sources that reach this wave's rows
+        const int mine = g + (lane & (kGB4 - 1));
+        const float mw = wl[mine].w;
+        const unsigned mu = (wl[mine].units >> (4 * wv)) & 15u;
+        unsigned mm = (unsigned)__ballot(lane < ng && mu != 0u);
+        __syncthreads();
+        const auto read = [&](int u, float2& x, float4& y) {
+          x = *reinterpret_cast<const float2*>(&fx_s[b][u][TR * wv + 2 * q]);
+          y = fy_s[b][u][c];
+        };
+        float2 xn = make_float2(0.f, 0.f);
+        float4 yn = make_float4(0.f, 0.f, 0.f, 0.f);
+        int u = mm ? __ffs((int)mm) - 1 : 0;
+        if (mm) read(u, xn, yn);
+        while (mm) {  // the next source's factors are read while this one is added
+          const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mw), u));
+          const float2 x = xn;
+          const float4 y4 = yn;
+          mm &= mm - 1;
+          if (mm) {
+            u = __ffs((int)mm) - 1;
+            read(u, xn, yn);
+          }
+          const float y[4] = {y4.x, y4.y, y4.z, y4.w};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            acc[0][k] = fmaf(x.x * y[k], w, acc[0][k]);
+            acc[1][k] = fmaf(x.y * y[k], w, acc[1][k]);
+          }
+        }
+      }
+    }
+  }
+  float a[TR], aA[TWO ? TR : 1];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    transpose_groups(acc[i]);
+    if constexpr (TWO) transpose_groups(accA[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[4 * i + j] = acc[i][j];
+      if constexpr (TWO) aA[4 * i + j] = accA[i][j];
+    }
+  }
+  double p[1][2];
+  tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out, p);
+  if (!spec.cm_out) return;
+  cm_s[wv][0][lane] = p[0][0];
+  cm_s[wv][1][lane] = p[0][1];
+  __syncthreads();
+  if (wv == 0) {
+    double s0 = p[0][0], s1 = p[0][1];
+    for (int v = 1; v < NW; ++v) {
+      s0 += cm_s[v][0][lane];
+      s1 += cm_s[v][1][lane];
+    }
+    tile_cm(cfg, at, s0, s1, spec.cm_out);
+  }
 }
 
-// The fused MC-KLN launch in the ctx's tile shape (the same shapes as
-// launch_tile; its centre-of-mass partials have tile_units(cfg) units).
+// The events of a batch by falling source count (64 classes), so that the
+// longest tiles start first and the batch ends without waiting for one of
+// them.  The order within a class is free: results do not depend on it.
+__global__ __launch_bounds__(1024) void k_tile_order(const int* __restrict__ counts, int nev, int top,
+                                                     int* __restrict__ order) {
+  __shared__ int cls[64], base[64];
+  const int t = threadIdx.x;
+  if (t < 64) cls[t] = 0;
+  __syncthreads();
+  const auto cls_of = [&](int e) { return 63 - min(63, (int)((long long)counts[(size_t)e * 8 + 5] * 64 / (top + 1))); };
+  for (int e = t; e < nev; e += 1024) atomicAdd(&cls[cls_of(e)], 1);
+  __syncthreads();
+  if (t == 0) {
+    int s = 0;
+    for (int k = 0; k < 64; ++k) {
+      base[k] = s;
+      s += cls[k];
+    }
+  }
+  __syncthreads();
+  for (int e = t; e < nev; e += 1024) order[atomicAdd(&base[cls_of(e)], 1)] = e;
+}
+
+// ---- sixteen waves per tile, for batches too small to fill the chip: a
+// tile's time is then the chain over its sources, a central event's the
+// longest (1,800 sources in one tile).  A wave owns 8 rows x 16 columns, one
+// unit of the selection, and adds only the sources that reach it.  The
+// workgroup selects 1024 sources at a time (the next 1024 are loaded
+// meanwhile) and computes the factors of kGB sources together, double-
+// buffered, one barrier per kGB sources.  The sums go through LDS to the four
+// waves that store the tile as the one-wave kernel does.
+constexpr int kGB = 32;
+
+template <int EPI>
+__global__ __launch_bounds__(1024) void k_tile16(DevCfg cfg, EvBufs buf, SmearSpec spec, int acc_sel, int nev,
+                                                 int spread, const int* order, float* out, KlnTab kt) {
+  constexpr int NW = 16, TR = 8, NT = 64 * NW;
+  constexpr bool TWO = EPI != 0;
+  __shared__ TileEntry wl[NT];
+  __shared__ float fx_s[2][kGB][kTileRows];  // K gx: row 8 v + q + 4 i at 8 v + 2 q + i
+  __shared__ float fy_s[2][kGB][64];         // gy
+  __shared__ int cnt_s[NW];
+  __shared__ float sum_s[TWO ? 2 : 1][kTileRows][64];
+  __shared__ double cm_s[4][2][64];
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), q = lane >> 4, c = lane & 15;
+  const int wr = wv >> 2, wc = wv & 3;  // the wave's 8 rows and 16 columns: unit 4 wr + wc = wv
+  const TileAt at = tile_at(cfg, buf, nev, spread, order);
+  if (at.e < 0) return;
+  const int e = at.e, R0 = at.R0, c0 = at.c0;
+  const bool live = at.col_live && at.x0 < R0 + kTileRows && at.x1 > R0;
+  if (!live && spec.sparse) {  // uniform over the workgroup
+    if (spec.cm_out && t < 4) spec.cm_out[((size_t)e * at.T + at.tile) * 4 + t] = 0.0;
+    return;
+  }
+  const float cq = cfg.inv2w2 * 1.4426950408889634f * (kHf * kHf);
+  const float kk = cfg.tile_k;
+  const int col = c0 + lane, row = R0 + (t & 31);  // of the factors this thread computes
+  const int ygh = (int)llrint((cfg.ymin + col * cfg.dy) / kH);
+  const int rowh = (int)llrint((cfg.xmin + row * cfg.dx) / kH);
+  const int fxi = (t & 24) + 2 * (t & 3) + ((t >> 2) & 1);
+  const int4* src = buf.src + (size_t)e * buf.src_cap;
+  const int4* swin = buf.swin + (size_t)e * buf.src_cap;
+
+  for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
+    float acc0 = 0.f, acc1 = 0.f;  // rows q and q + 4 of the wave's 8
+    const int want = TWO ? pass : acc_sel;
+    const int2 kr = source_range(buf, spec, e, want);
+    const int k0 = kr.x, K = live ? kr.y : 0;
+    int4 ps = make_int4(0, 0, 0, 0), pw = ps;  // this thread's source of the next 1024
+    if (k0 + t < K) {
+      ps = src[k0 + t];
+      pw = swin[k0 + t];
+    }
+    for (int sub = k0; sub < K; sub += NT) {
+      TileEntry en{0, 0, 0, 0, 0.f, 0u};
+      if (sub + t < K) en = tile_entry<TR, 4>(cfg, spec, ps, pw, want, R0, c0);
+      if (sub + NT + t < K) {
+        ps = src[sub + NT + t];
+        pw = swin[sub + NT + t];
+      }
+      const unsigned long long m = __ballot(en.units != 0u);
+      __syncthreads();  // the entries and counts of the last round are read
+      if (lane == 0) cnt_s[wv] = __popcll(m);
+      __syncthreads();
+      int n = 0, at_n = 0;
+#pragma unroll
+      for (int v = 0; v < NW; ++v) {
+        if (v == wv) at_n = n;
+        n += cnt_s[v];
+      }
+      if (en.units) wl[at_n + __popcll(m & ((1ull << lane) - 1ull))] = en;
+      __syncthreads();
+      for (int g = 0; g < n; g += kGB) {
+        const int b = (g / kGB) & 1, ng = min(kGB, n - g);
+        // factors: rows of 32 sources in one pass, columns of 16 per pass
+        {
+          const int s = t >> 5;
+          if (s < ng) {
+            const int2 ex = *reinterpret_cast<const int2*>(&wl[g + s].xh);
+            const float dx = (float)(rowh - ex.x);
+            const int xlo = ex.y & 0xffff, xhi = ex.y >> 16;
+            const float gx = kk * __builtin_amdgcn_exp2f(-(dx * dx) * cq);
+            fx_s[b][s][fxi] = (row >= xlo && row < xhi) ? gx : 0.f;
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < kGB; p += NW) {
+          const int s = p + wv;
+          if (s < ng) {
+            const int2 ey = *reinterpret_cast<const int2*>(&wl[g + s].yh);
+            const float dy = (float)(ygh - ey.x);
+            const int ylo = ey.y & 0xffff, yhi = ey.y >> 16;
+            fy_s[b][s][lane] = (col >= ylo && col < yhi) ? __builtin_amdgcn_exp2f(-(dy * dy) * cq) : 0.f;
+          }
+        }
+        // the batch's sources that reach this wave's unit
+        const int mine = g + (lane & (kGB - 1));
+        const float mw = wl[mine].w;
+        unsigned mm = (unsigned)__ballot(lane < ng && ((wl[mine].units >> wv) & 1u));
+        __syncthreads();
+        while (mm) {  // four sources' factors are read before they are added, in order
+          float2 x[4];
+          float y[4], w[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            if (mm) {
+              const int u = __ffs((int)mm) - 1;
+              mm &= mm - 1;
+              x[v] = *reinterpret_cast<const float2*>(&fx_s[b][u][TR * wr + 2 * q]);
+              y[v] = fy_s[b][u][16 * wc + c];
+              w[v] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mw), u));
+            } else {
+              x[v] = make_float2(0.f, 0.f);
+              y[v] = w[v] = 0.f;
+            }
+          }
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            acc0 = fmaf(x[v].x * y[v], w[v], acc0);
+            acc1 = fmaf(x[v].y * y[v], w[v], acc1);
+          }
+        }
+      }
+    }
+    sum_s[TWO ? pass : 0][TR * wr + q][16 * wc + c] = acc0;
+    sum_s[TWO ? pass : 0][TR * wr + q + 4][16 * wc + c] = acc1;
+  }
+  __syncthreads();
+  if (wv < 4) {  // wave v stores rows 8 v .. 8 v + 7
+    const int r0 = R0 + TR * wv;
+    float a[TR], aA[TWO ? TR : 1];
+#pragma unroll
+    for (int r = 0; r < TR; ++r) {
+      a[r] = sum_s[TWO ? 1 : 0][TR * wv + r][lane];
+      if constexpr (TWO) aA[r] = sum_s[0][TR * wv + r][lane];
+    }
+    double p[1][2];
+    tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out, p);
+    cm_s[wv][0][lane] = p[0][0];
+    cm_s[wv][1][lane] = p[0][1];
+  }
+  if (!spec.cm_out) return;
+  __syncthreads();
+  if (wv == 0) {
+    double s0 = cm_s[0][0][lane], s1 = cm_s[0][1][lane];
+    for (int v = 1; v < 4; ++v) {
+      s0 += cm_s[v][0][lane];
+      s1 += cm_s[v][1][lane];
+    }
+    tile_cm(cfg, at, s0, s1, spec.cm_out);
+  }
+}
+
+int tile_units(const DevCfg& cfg) { return ((cfg.nx + kTileRows - 1) / kTileRows) * ((cfg.ny + 63) / 64); }
+
+// Waves per tile.  Variants 1, 2, 3 (smc_set_tile_variant) are one, four and
+// sixteen; 0 chooses by the number of tiles and by whether the lists hold the
+// collision pairs (a central Pb+Pb list is then 2,000 sources long, else 400).
+// Per batch of Pb+Pb events of 261^2 cells (45 tiles), us with 1 / 4 / 16 waves:
+//   with pairs      1 event 282 / 141 / 72, 128 472 / 239 / 145, 256 482 / 243 / 261,
+//                   1000 504 / 362 / 1013, 2000 560 / 694 / 2018
+//   MC-KLN, sqrt    1 event 67 / 33 / 20, 64 95 / 48 / 63, 512 106 / 111 / 389,
+//                   1000 167 / 198 / 725
+static int waves_of(const DevCfg& cfg, const SmearSpec& s, int nev) {
+  constexpr int kWaves[kTileVariants] = {0, 1, 4, 16};
+  if (cfg.tile_variant > 0 && cfg.tile_variant < kTileVariants) return kWaves[cfg.tile_variant];
+  const long long tiles = (long long)tile_units(cfg) * nev;
+  const bool pairs = s.enabled[kSrcPair];
+  return tiles <= (pairs ? 9000 : 2200) ? 16 : (tiles <= (pairs ? 58000 : 20000) ? 4 : 1);
+}
+
+// Longest events first: 1000 events 735 -> 504 us with one wave per tile, 543 ->
+// 362 with four; 16,000 events 3.2 -> 2.9 ms.  One workgroup orders 32,768
+// events in about 60 us; larger batches lose less to their last tiles.
+static bool ordered(int nev) { return nev >= 16 && nev <= 32768; }
+
+template <int EPI>
+static void launch_shape(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int acc_sel, int nev, float* out,
+                         const KlnTab& kt, hipStream_t st) {
+  const int waves = waves_of(cfg, s, nev);
+  const int spread = nev < 64;  // 8 events per XCD keep its 32 CUs busy
+  const int* order = ordered(nev) ? b.order : nullptr;
+  // one dimension: tiles x events; with an event's tiles on one XCD, events
+  // padded to a multiple of the 8 XCDs
+  const dim3 grid((unsigned)tile_units(cfg) * (spread ? (unsigned)nev : (unsigned)((nev + 7) / 8 * 8)));
+  if (waves == 16)
+    hipLaunchKernelGGL(k_tile16<EPI>, grid, dim3(1024), 0, st, cfg, b, s, acc_sel, nev, spread, order, out, kt);
+  else if (waves == 4)
+    hipLaunchKernelGGL(k_tile4<EPI>, grid, dim3(256), 0, st, cfg, b, s, acc_sel, nev, spread, order, out, kt);
+  else
+    hipLaunchKernelGGL(k_tile<EPI>, grid, dim3(64), 0, st, cfg, b, s, acc_sel, nev, spread, order, out, kt);
+}
+
+static void launch_order(const EvBufs& b, int nev, hipStream_t st) {
+  if (ordered(nev)) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, st, b.counts, nev, 2048, b.order);
+}
+
+// The fused MC-KLN launch (its centre-of-mass partials have tile_units(cfg)
+// units).
 int launch_tile_kln(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev, float* out,
                     const double* table, int tmax, double dT, void* stream) {
   if (nev <= 0) return 0;
   if (!(cfg.tile_k > 0.f && cfg.tile_w > 0.f && cfg.tile_out > 0.f) || !table || tmax < 3 || !(dT > 0))
     return (int)hipErrorInvalidValue;
-  const KlnTab kt{table, tmax, dT};
-  hipStream_t st = (hipStream_t)stream;
-  switch (variant_of(cfg)) {
-    case 1: launch_tr_kln<16, 8, true>(cfg, b, s, nev, out, kt, st); break;
-    case 2: launch_tr_kln<32, 4, true>(cfg, b, s, nev, out, kt, st); break;
-    case 3: launch_tr_kln<64, 8, false>(cfg, b, s, nev, out, kt, st); break;
-    default: launch_tr_kln<kTileRows, 8, true>(cfg, b, s, nev, out, kt, st); break;
-  }
+  launch_order(b, nev, (hipStream_t)stream);
+  launch_shape<1>(cfg, b, s, 0, nev, out, KlnTab{table, tmax, dT}, (hipStream_t)stream);
   return (int)hipGetLastError();
 }
 
@@ -342,12 +814,16 @@ int launch_tile(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev,
   if (nev <= 0) return 0;
   if (!(cfg.tile_k > 0.f && cfg.tile_w > 0.f && cfg.tile_out > 0.f)) return (int)hipErrorInvalidValue;
   hipStream_t st = (hipStream_t)stream;
-  switch (variant_of(cfg)) {
-    case 1: launch_tr<16, 8, true>(cfg, b, s, nev, out0, out1, st); break;
-    case 2: launch_tr<32, 4, true>(cfg, b, s, nev, out0, out1, st); break;
-    case 3: launch_tr<64, 8, false>(cfg, b, s, nev, out0, out1, st); break;
-    default: launch_tr<kTileRows, 8, true>(cfg, b, s, nev, out0, out1, st); break;
+  const KlnTab none{nullptr, 0, 1.0};
+  launch_order(b, nev, st);
+  if (s.combine == 1) {  // sqrt(T_A T_B) in one launch, with the partials of the combined grid
+    launch_shape<2>(cfg, b, s, 0, nev, out0, none, st);
+    return (int)hipGetLastError();
   }
+  SmearSpec s1 = s;  // partials only for a single accumulator
+  if (s.combine != 0) s1.cm_out = nullptr;
+  launch_shape<0>(cfg, b, s1, 0, nev, out0, none, st);
+  if (s.combine != 0) launch_shape<0>(cfg, b, s1, 1, nev, out1, none, st);
   return (int)hipGetLastError();
 }
 
