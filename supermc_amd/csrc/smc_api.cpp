@@ -1660,8 +1660,11 @@ smc_status smc_density_f64(smc_ctx* c, int ev0, int n, double* s) {
     Grid64Const gc{};
     gc.norm = 1 / (2 * M_PI * w * w);
     gc.two_w_w = 2 * w * w;
-    gc.two_wsq = 2 * wsq;
-    gc.r_max = 5 * w;
+    // the largest double whose root is at most 5 w (sqrt rounds monotonically)
+    const double r_max = 5 * w;
+    gc.part_max = r_max * r_max;
+    while (std::sqrt(gc.part_max) > r_max) gc.part_max = std::nextafter(gc.part_max, 0.0);
+    while (std::sqrt(std::nextafter(gc.part_max, HUGE_VAL)) <= r_max) gc.part_max = std::nextafter(gc.part_max, HUGE_VAL);
     gc.dc_max = 25. * wsq;
     gc.alpha = c->p.alpha;
     gc.prefactor = (1.0 - c->p.alpha) / 2.;

@@ -5,146 +5,177 @@
 // Particle::getSmoothDensity (Particle.cpp:122-132, 168-174) over their
 // boxes, collisions over the +-5w windows with the dc <= 25 w^2 cut.
 //
-// Per (source, cell) in FP64, as the reference writes it:
-//   participant  r = sqrt((xg-x)^2 + (yg-y)^2); r > 5w -> 0, else
-//                (1/(2 pi w^2)) exp(-r r / (2 w w)), times f
-//   collision    dc = (x-xg)^2 + (y-yg)^2 <= 25 w^2:
-//                f (1/(2 pi w^2)) exp(-dc / (2 w^2)) (alpha + (1 - alpha) aw)
-//                with aw = 0, or for sub_model 2 (MCnucl.cpp:713-717: no
-//                participant term) the pair's weight of MCnucl.cpp:345-348
-// summed per cell in source order (participants of A and B in wound order,
-// then the pairs in pair order), the participant sum scaled by (1-alpha)/2
-// at the end.  The file is built with -ffp-contract=off so that no product
-// and sum fuse: every operation rounds as the reference's x86-64 doubles do,
-// and only exp may differ from the host's by an ulp.
+// Per (source, cell) in FP64:
+//   participant  f / (2 pi w^2) exp(-d^2 / 2w^2) where sqrt(d^2) <= 5w,
+//   collision    f / (2 pi w^2) exp(-d^2 / 2w^2) (alpha + (1 - alpha) aw) where
+//                d^2 <= 25 w^2, with aw = 0, or for sub_model 2
+//                (MCnucl.cpp:713-717: no participant term) the pair's weight
+//                of MCnucl.cpp:345-348,
+// d^2 = dx^2 + dy^2 rounded as the reference's x86-64 doubles round it (the file
+// is built with -ffp-contract=off), so both cuts take the reference's cells:
+// sqrt(d^2) <= 5w is the compare d^2 <= part_max with the largest double whose
+// root passes (host).  The exponential factorises, exp(-dx^2/2w^2)
+// exp(-dy^2/2w^2): a cell costs an add, a compare and an FMA under its mask
+// instead of a square root, a division and an exponential, and stays within a
+// few ulp of the undivided form.  Terms are added in source order (participants
+// of A and B in wound order, then the pairs in pair order), the weights f
+// norm (1 - alpha)/2 and f norm alpha folded into the column factors.
 //
-// One workgroup of 4 waves per (16 x 64 tile, event); lane = column, each
-// wave 4 rows.  Tiles outside the event's source rectangle are written as
-// zeros without a source pass.
+// One workgroup of 4 waves per (32 x 64 tile, event), a wave 8 rows, laid out as
+// k_tile4 of smc_tile.hip: lane (q, c) holds rows q, q + 4 and columns c + 16 k;
+// the workgroup selects 256 sources at a time and shares the factors of 8.
+// Bound by the factors' exponentials and VALU issue about equally: 250 Au+Au
+// events of 261^2 cells 497 us (2226 us with an exponential per term).
+// Tiles outside the event's source rectangle are written as zeros without a
+// source pass.
 #include "smc_device.h"
 
 namespace smc {
 
 namespace {
-constexpr int kGX = 16, kGY = 64;
-}
+constexpr int kGX = 32, kGY = 64, kG64 = 8;
 
+struct Entry64 {
+  int xh, xw, yh, yw;
+  double w;
+  int pair, chunks;  // chunks: the 8-row chunks of the tile that the window meets
+};
+}  // namespace
+
+template <bool TWO>
 __global__ __launch_bounds__(256) void k_grid64(DevCfg cfg, EvBufs buf, Grid64Const gc, int ev0, double* out) {
-  const int el = blockIdx.y;
-  const int e = ev0 + el;
+  constexpr int NW = 4, TR = kGX / NW;
+  __shared__ Entry64 wl[256];
+  __shared__ double2 fx_s[2][kG64][kGX];  // {gx, dx^2}: row 8 v + q + 4 i at 8 v + 2 q + i
+  __shared__ double2 fy_s[2][kG64][kGY];  // {w gy, dy^2}
+  __shared__ int cnt_s[NW];
+  const int el = blockIdx.y, e = ev0 + el;
   const int ntx = (cfg.nx + kGX - 1) / kGX;
-  const int tx0 = (blockIdx.x % ntx) * kGX, ty0 = (blockIdx.x / ntx) * kGY;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int iy = ty0 + lane;
-  const int rx0 = tx0 + wv * 4;
-
-  __shared__ double2 lpos[256];
-  __shared__ int4 lwin[256];  // x lo, x hi, y lo, y hi
-  __shared__ double lf[256];
-  __shared__ double lw[256];  // pair weight: alpha, or alpha + (1 - alpha) aw for sub_model 2
-  __shared__ int lacc[256];   // 0: participant sum, 1: collision sum / nucleus B
-  __shared__ int lpair[256];  // 1: collision term
-  __shared__ int wcount[4];
-
+  const int R0 = (blockIdx.x % ntx) * kGX, c0 = (blockIdx.x / ntx) * kGY;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), q = lane >> 4, c = lane & 15;
   const int rxp = buf.counts[(size_t)e * 8 + 6], ryp = buf.counts[(size_t)e * 8 + 7];
-  const bool live = tx0 < (rxp >> 16) && tx0 + kGX > (rxp & 0xffff) && ty0 < (ryp >> 16) &&
-                    ty0 + kGY > (ryp & 0xffff);
-
-  double xg[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) xg[r] = cfg.xmin + (double)(rx0 + r) * cfg.dx;
-  const double yg = cfg.ymin + (double)iy * cfg.dy;
-
-  double a0[4] = {0.0, 0.0, 0.0, 0.0}, a1[4] = {0.0, 0.0, 0.0, 0.0};
+  const bool live = R0 < (rxp >> 16) && R0 + kGX > (rxp & 0xffff) && c0 < (ryp >> 16) && c0 + kGY > (ryp & 0xffff);
+  const int npa = buf.counts[(size_t)e * 8], npart = npa + buf.counts[(size_t)e * 8 + 1];
   const int K = live ? buf.counts[(size_t)e * 8 + 5] : 0;  // uniform over the workgroup
-  const int nsrc_part = buf.counts[(size_t)e * 8] + buf.counts[(size_t)e * 8 + 1];
-  const size_t pbase = (size_t)e * cfg.max_pairs;
   const int4* src = buf.src + (size_t)e * buf.src_cap;
   const int4* swin = buf.swin + (size_t)e * buf.src_cap;
+  const size_t pbase = (size_t)e * cfg.max_pairs;
+  const int row = R0 + (t & 31), col = c0 + lane;  // of the factors this thread computes
+  const double xg = cfg.xmin + (double)row * cfg.dx, yg = cfg.ymin + (double)col * cfg.dy;
+  const int fxi = (t & 24) + 2 * (t & 3) + ((t >> 2) & 1);
 
-  for (int base = 0; base < K; base += 256) {
-    const int k = base + t;
-    bool take = false;
-    double2 pos = make_double2(0.0, 0.0);
-    int4 win = make_int4(0, 0, 0, 0);
-    double f = 1.0, wgt = gc.alpha;
-    int acc = 0, pair = 0;
-    if (k < K) {
-      const int4 s = src[k];
-      const int4 w4 = swin[k];
-      pair = s.w == kSrcPair;
-      const int wx = pair ? w4.z : w4.x, wy = pair ? w4.w : w4.y;  // 5w windows for collisions, boxes otherwise
-      win = make_int4(wx & 0xffff, wx >> 16, wy & 0xffff, wy >> 16);
-      take = (pair ? gc.use_binary : !gc.uli) && win.x < win.y && win.z < win.w && win.x < tx0 + kGX &&
-             win.y > tx0 && win.z < ty0 + kGY && win.w > ty0;
-      pos = make_double2((double)s.x * kH, (double)s.y * kH);
-      f = gc.fluct ? (double)__int_as_float(s.z) : 1.0;
-      if (pair && gc.uli) {  // the pair's Gamma factor and (Alpha + (1 - Alpha) aw) of MCnucl.cpp:755
-        const size_t pk = pbase + (size_t)(k - nsrc_part);
-        f = gc.fluct ? (double)buf.pfluct[pk] : 1.0;
-        wgt = gc.alpha + (1. - gc.alpha) * (double)buf.paw[pk];
-      }
-      acc = gc.model == 7 ? (s.w == kSrcPartB) : pair;
-    }
-    // ordered compaction: the tile's sources in list order
-    const unsigned long long m = __ballot(take);
-    const int before = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) wcount[wv] = __popcll(m);
-    __syncthreads();
-    int woff = 0;
-    for (int q = 0; q < wv; ++q) woff += wcount[q];
-    const int n = wcount[0] + wcount[1] + wcount[2] + wcount[3];
-    if (take) {
-      lpos[woff + before] = pos;
-      lwin[woff + before] = win;
-      lf[woff + before] = f;
-      lw[woff + before] = wgt;
-      lacc[woff + before] = acc;
-      lpair[woff + before] = pair;
-    }
-    __syncthreads();
-    for (int q = 0; q < n; ++q) {
-      const int4 ww = lwin[q];
-      if (rx0 >= ww.y || rx0 + 4 <= ww.x) continue;  // wave-uniform
-      if (iy < ww.z || iy >= ww.w) continue;
-      const double2 p = lpos[q];
-      const double fq = lf[q];
-      const bool to1 = lacc[q] != 0;
-      if (lpair[q]) {
+  double acc[2][4], accA[TWO ? 2 : 1][4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int ix = rx0 + r;
-          if (ix < ww.x || ix >= ww.y) continue;
-          const double ddx = p.x - xg[r], ddy = p.y - yg;
-          const double dc = ddx * ddx + ddy * ddy;
-          if (dc <= gc.dc_max) {
-            const double v = fq * gc.norm * exp(-dc / gc.two_wsq) * lw[q];
-            if (to1) a1[r] += v; else a0[r] += v;
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[i][k] = 0.0;
+  for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
+    if (TWO && pass == 1) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          accA[TWO ? i : 0][k] = acc[i][k];
+          acc[i][k] = 0.0;
+        }
+    }
+    // model 7: the projectile's participants, then the target's; model 5: the
+    // whole list, without the pairs at alpha = 0 and without the
+    // participants for sub_model 2
+    const int k0 = TWO ? (pass ? min(npa, K) : 0) : (gc.uli ? min(npart, K) : 0);
+    const int k1 = TWO ? min(pass ? npart : npa, K) : (gc.use_binary ? K : min(npart, K));
+    for (int sub = k0; sub < k1; sub += 256) {
+      const int k = sub + t;
+      Entry64 en{0, 0, 0, 0, 0.0, 0, 0};
+      if (k < k1) {
+        const int4 s = src[k];
+        const int4 w4 = swin[k];
+        en.pair = s.w == kSrcPair;
+        en.xh = s.x;
+        en.yh = s.y;
+        en.xw = en.pair ? w4.z : w4.x;  // 5w windows for collisions, boxes otherwise
+        en.yw = en.pair ? w4.w : w4.y;
+        double f = gc.fluct ? (double)__int_as_float(s.z) : 1.0;
+        double m = en.pair ? gc.alpha : (TWO ? 1.0 : gc.prefactor);
+        if (en.pair && gc.uli) {  // the pair's Gamma factor and (Alpha + (1 - Alpha) aw) of MCnucl.cpp:755
+          const size_t pk = pbase + (size_t)(k - npart);
+          f = gc.fluct ? (double)buf.pfluct[pk] : 1.0;
+          m = gc.alpha + (1. - gc.alpha) * (double)buf.paw[pk];
+        }
+        en.w = f * gc.norm * m;
+        const int xlo = en.xw & 0xffff, xhi = en.xw >> 16, ylo = en.yw & 0xffff, yhi = en.yw >> 16;
+        if (xlo < xhi && ylo < yhi && ylo < c0 + kGY && yhi > c0)
+#pragma unroll
+          for (int v = 0; v < NW; ++v)
+            if (xlo < R0 + TR * (v + 1) && xhi > R0 + TR * v) en.chunks |= 1 << v;
+      }
+      // ordered compaction: the tile's sources in list order
+      const unsigned long long m = __ballot(en.chunks != 0);
+      __syncthreads();  // the entries and counts of the last round are read
+      if (lane == 0) cnt_s[wv] = __popcll(m);
+      __syncthreads();
+      int n = 0, at_n = 0;
+#pragma unroll
+      for (int v = 0; v < NW; ++v) {
+        if (v == wv) at_n = n;
+        n += cnt_s[v];
+      }
+      if (en.chunks) wl[at_n + __popcll(m & ((1ull << lane) - 1ull))] = en;
+      __syncthreads();
+      for (int g = 0; g < n; g += kG64) {
+        const int b = (g / kG64) & 1, ng = min(kG64, n - g);
+        {  // rows of the 8 sources, then columns of 4 sources per pass
+          const int s = t >> 5;
+          if (s < ng) {
+            const int xw = wl[g + s].xw;
+            const double d = xg - (double)wl[g + s].xh * kH, d2 = d * d;
+            const bool in = row >= (xw & 0xffff) && row < (xw >> 16);
+            fx_s[b][s][fxi] = make_double2(in ? exp(-d2 / gc.two_w_w) : 0.0, d2);
           }
         }
-      } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int ix = rx0 + r;
-          if (ix < ww.x || ix >= ww.y) continue;
-          const double ddx = xg[r] - p.x, ddy = yg - p.y;
-          const double rr = sqrt(ddx * ddx + ddy * ddy);
-          const double tn = (rr > gc.r_max) ? 0.0 : gc.norm * exp(-rr * rr / gc.two_w_w);
-          const double v = tn * fq;
-          if (to1) a1[r] += v; else a0[r] += v;
+        for (int p = 0; p < kG64; p += NW) {
+          const int s = p + wv;
+          if (s < ng) {
+            const int yw = wl[g + s].yw;
+            const double d = yg - (double)wl[g + s].yh * kH, d2 = d * d;
+            const bool in = col >= (yw & 0xffff) && col < (yw >> 16);
+            fy_s[b][s][lane] = make_double2(in ? wl[g + s].w * exp(-d2 / gc.two_w_w) : 0.0, d2);
+          }
+        }
+        const int mine = g + (lane & (kG64 - 1));
+        unsigned mm = (unsigned)__ballot(lane < ng && ((wl[mine].chunks >> wv) & 1));
+        const unsigned pm = (unsigned)__ballot(lane < ng && wl[mine].pair);
+        __syncthreads();
+        while (mm) {
+          const int u = __ffs((int)mm) - 1;
+          mm &= mm - 1;
+          const double cut = ((pm >> u) & 1u) ? gc.dc_max : gc.part_max;
+          double2 x[2], y[4];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) x[i] = fx_s[b][u][TR * wv + 2 * q + i];
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) y[kk] = fy_s[b][u][16 * kk + c];
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+              if (x[i].y + y[kk].y <= cut) acc[i][kk] = fma(x[i].x, y[kk].x, acc[i][kk]);
         }
       }
     }
-    __syncthreads();
   }
-  if (iy >= cfg.ny) return;
   const size_t N = (size_t)cfg.nx * cfg.ny;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int ix = rx0 + r;
+  for (int i = 0; i < 2; ++i) {
+    const int ix = R0 + TR * wv + q + 4 * i;
     if (ix >= cfg.nx) continue;
-    const double v = gc.model == 7 ? sqrt(a0[r] * a1[r]) : a0[r] * gc.prefactor + a1[r];
-    out[(size_t)el * N + (size_t)ix * cfg.ny + iy] = v;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int iy = c0 + c + 16 * k;
+      if (iy < cfg.ny)
+        out[(size_t)el * N + (size_t)ix * cfg.ny + iy] = TWO ? sqrt(accA[TWO ? i : 0][k] * acc[i][k]) : acc[i][k];
+    }
   }
 }
 
@@ -152,7 +183,10 @@ int launch_grid64(const DevCfg& cfg, const EvBufs& b, const Grid64Const& gc, int
                   void* stream) {
   if (nev <= 0) return 0;
   const int ntx = (cfg.nx + kGX - 1) / kGX, nty = (cfg.ny + kGY - 1) / kGY;
-  hipLaunchKernelGGL(k_grid64, dim3(ntx * nty, nev), dim3(256), 0, (hipStream_t)stream, cfg, b, gc, ev0, out);
+  if (gc.model == 7)
+    hipLaunchKernelGGL(k_grid64<true>, dim3(ntx * nty, nev), dim3(256), 0, (hipStream_t)stream, cfg, b, gc, ev0, out);
+  else
+    hipLaunchKernelGGL(k_grid64<false>, dim3(ntx * nty, nev), dim3(256), 0, (hipStream_t)stream, cfg, b, gc, ev0, out);
   return (int)hipGetLastError();
 }
 

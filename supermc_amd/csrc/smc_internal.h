@@ -170,14 +170,12 @@ struct SmearSpec {
                     // launch_zero_outside first); 0: whole grids are written
 };
 
-// FP64 density grids (smc_grid64.hip): the reference's double expressions,
-// evaluated per (source, cell); constants computed on the host as the
+// FP64 density grids (smc_grid64.hip); constants computed on the host as the
 // reference writes them
 struct Grid64Const {
   double norm;       // 1 / (2 pi w w)
-  double two_w_w;    // 2 w w   (Particle.cpp:122-132)
-  double two_wsq;    // 2 (w w) (MCnucl.cpp:732-756)
-  double r_max;      // 5 w
+  double two_w_w;    // 2 w w   (Particle.cpp:122-132, MCnucl.cpp:732-756)
+  double part_max;   // the largest d^2 with sqrt(d^2) <= 5 w
   double dc_max;     // 25 (w w)
   double alpha, prefactor;  // alpha, (1 - alpha) / 2
   int model;         // which_mc_model: 5 or 7

@@ -98,3 +98,25 @@ def test_fp64_grid_ranges_and_chunks_are_event_local():
         with pytest.raises(SmcError) as ei:
             ctx.density_f64()
         assert ei.value.code == SMC_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("model", [5, 7])
+@pytest.mark.parametrize("maxx,maxy,dx", [(4.0, 4.0, 0.125), (3.3, 0.8, 0.1), (0.7, 6.4, 0.1)])
+def test_fp64_grid_edges_and_cells_on_the_cut(model, maxx, maxy, dx):
+    """Partial tiles in both directions (65 x 65, 67 x 17, 15 x 129 cells) and
+    nucleons on grid points of 0.125 fm, where cells lie at exactly 5 w = 2.5
+    fm (20 cells along an axis, 12 and 16 across): the same cells as the
+    oracle's are non-zero, and their values agree to the 1e-12 bar."""
+    from supermc_amd import Context
+    p = H.glauber_params("PbPb", Aproj=3 + 2, Atarg=5, max_events=2, which_mc_model=model, maxx=maxx, maxy=maxy, dx=dx,
+                         dy=dx, cc_fluctuation_model=0)
+    xa = np.array([[[0.0, 0.0], [0.5, 0.25], [-0.25, 0.125], [0.375, -0.5], [1.5, 0.0]]] * 2)
+    xb = np.array([[[0.0, 0.0], [0.25, 0.5], [-0.5, -0.125], [0.125, 0.0], [2.0, 0.25]]] * 2)
+    xb[1, :, 1] += 0.125
+    with Context(p) as ctx:
+        ctx.set_positions(xa, xb)
+        s = ctx.density_f64()
+        for e in range(2):
+            o = H.oracle_event(ctx, e)
+            assert np.array_equal(s[e] != 0.0, o["s"] != 0.0)
+            assert H.rel_linf(s[e], o["s"]) <= TOL64
