@@ -29,7 +29,7 @@ KERNEL_SOURCES = ["smc_kernels.hip", "smc_moments.hip", "smc_mtile.hip", "smc_ti
 # takes minima of node values without NaN quieting (finite inputs only).
 SOURCE_FLAGS = {"smc_tile.hip": ["-fgpu-flush-denormals-to-zero"], "smc_grid64.hip": ["-ffp-contract=off"],
                 "smc_kln_direct.hip": ["-fno-honor-nans"]}
-HOST_SOURCES = ["smc_api.cpp", "smc_p3d_api.cpp"]
+HOST_SOURCES = ["smc_api.cpp", "smc_p3d_api.cpp", "smc_copy.cpp"]
 
 
 def _run(cmd):

@@ -12,6 +12,7 @@
 #include <string>
 #include <vector>
 
+#include "smc_copy.h"
 #include "smc_internal.h"
 
 using namespace smc;
@@ -161,6 +162,7 @@ struct smc_ctx {
   double* evout_alt = nullptr;
   double* stage[2] = {nullptr, nullptr};
   hipStream_t copy_stream = nullptr;
+  HostCopier copier;                 // grids and records into pageable memory
   hipEvent_t ev_done[2] = {nullptr, nullptr}, ev_copied[2] = {nullptr, nullptr};
   int* dtab = nullptr;
   float* grid = nullptr;
@@ -611,6 +613,13 @@ float* grid_buffer(smc_ctx* c, float** slot) {
 }
 
 void sync(smc_ctx* c) { HIPCHK(hipStreamSynchronize(c->stream)); }
+
+// device memory to the caller's, after the work on the ctx's stream; sync(c)
+// completes it
+void to_host(smc_ctx* c, void* dst, const void* src, size_t bytes) {
+  HIPCHK(c->copier.copy(dst, src, bytes, c->stream));
+}
+
 
 SmearSpec density_spec(const smc_ctx* c) {
   const DevCfg& g = c->cfg;
@@ -1614,8 +1623,8 @@ smc_status smc_thickness(smc_ctx* c, float* TA, float* TB) {
     run_smear(c, thickness_spec(c), a, b);
     c->have_thickness = 1;
     const size_t n = (size_t)c->nev * c->d.nx * c->d.ny;
-    if (TA) HIPCHK(hipMemcpyAsync(TA, a, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    if (TB) HIPCHK(hipMemcpyAsync(TB, b, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+    if (TA) to_host(c, TA, a, n * sizeof(float));
+    if (TB) to_host(c, TB, b, n * sizeof(float));
     sync(c);
     return SMC_OK;
   } catch (const SmcError& e) { return fail(c, e); }
@@ -1628,7 +1637,7 @@ smc_status smc_density(smc_ctx* c, float* s, double* dndy) {
     const size_t n = (size_t)c->nev * c->d.nx * c->d.ny;
     if (s) {
       densify_grid(c);
-      HIPCHK(hipMemcpyAsync(s, c->grid, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+      to_host(c, s, c->grid, n * sizeof(float));
     }
     int st = SMC_OK;
     if (dndy) {
@@ -1688,8 +1697,7 @@ smc_status smc_density_f64(smc_ctx* c, int ev0, int n, double* s) {
       TimerScope ts(c, SMC_K_GRID64);
       check_launch(launch_grid64(c->cfg, c->buf, gc, ev0 + e, m, c->grid64, c->stream), "k_grid64");
       ts.done();
-      HIPCHK(hipMemcpyAsync(s + (size_t)e * N, c->grid64, (size_t)m * N * sizeof(double), hipMemcpyDeviceToHost,
-                            c->stream));
+      to_host(c, s + (size_t)e * N, c->grid64, (size_t)m * N * sizeof(double));
     }
     sync(c);
     return SMC_OK;
@@ -1703,8 +1711,7 @@ smc_status smc_moments(smc_ctx* c, double* ev_out) {
     run_moments(c, 0);
     c->have_moments = 1;
     if (ev_out)
-      HIPCHK(hipMemcpyAsync(ev_out, c->evout, (size_t)c->nev * SMC_EV_STRIDE * sizeof(double),
-                            hipMemcpyDeviceToHost, c->stream));
+      to_host(c, ev_out, c->evout, (size_t)c->nev * SMC_EV_STRIDE * sizeof(double));
     sync(c);
     tag_systems(c, ev_out, c->nev);
     return SMC_OK;
@@ -1718,8 +1725,7 @@ smc_status smc_rho_binary(smc_ctx* c, float* rho) {
     float* g = grid_buffer(c, &c->aux0);
     run_rho_binary(c, g);
     if (rho)
-      HIPCHK(hipMemcpyAsync(rho, g, (size_t)c->nev * c->d.nx * c->d.ny * sizeof(float), hipMemcpyDeviceToHost,
-                            c->stream));
+      to_host(c, rho, g, (size_t)c->nev * c->d.nx * c->d.ny * sizeof(float));
     sync(c);
     return SMC_OK;
   } catch (const SmcError& e) { return fail(c, e); }
@@ -1733,8 +1739,8 @@ smc_status smc_spectator_density(smc_ctx* c, float* spec_proj, float* spec_targ)
     float* b = grid_buffer(c, &c->aux1);
     run_spectator_density(c, a, b);
     const size_t n = (size_t)c->nev * c->d.nx * c->d.ny * sizeof(float);
-    if (spec_proj) HIPCHK(hipMemcpyAsync(spec_proj, a, n, hipMemcpyDeviceToHost, c->stream));
-    if (spec_targ) HIPCHK(hipMemcpyAsync(spec_targ, b, n, hipMemcpyDeviceToHost, c->stream));
+    if (spec_proj) to_host(c, spec_proj, a, n);
+    if (spec_targ) to_host(c, spec_targ, b, n);
     sync(c);
     return SMC_OK;
   } catch (const SmcError& e) { return fail(c, e); }
@@ -1766,8 +1772,7 @@ smc_status smc_run(smc_ctx* c, uint64_t seed, uint64_t event0, int nev, double* 
     run_moments(c, 0);
     c->have_moments = 1;
     if (ev_out) {
-      HIPCHK(hipMemcpyAsync(ev_out, c->evout, (size_t)nev * SMC_EV_STRIDE * sizeof(double),
-                            hipMemcpyDeviceToHost, c->stream));
+      to_host(c, ev_out, c->evout, (size_t)nev * SMC_EV_STRIDE * sizeof(double));
       sync(c);
       tag_systems(c, ev_out, nev);
     }
@@ -1911,7 +1916,7 @@ smc_status smc_run_stream(smc_ctx* c, uint64_t seed, uint64_t event0, int64_t ne
       const int k = (int)(i & 1);
       HIPCHK(hipEventSynchronize(c->ev_copied[k]));
       double* dst = ev_out + (size_t)(i * cap) * SMC_EV_STRIDE;
-      std::memcpy(dst, c->stage[k], (size_t)nbatch[k] * rec);
+      parallel_memcpy(dst, c->stage[k], (size_t)nbatch[k] * rec);
       if (!c->mix_of.empty())
         for (int e = 0; e < nbatch[k]; ++e)
           dst[(size_t)e * SMC_EV_STRIDE + SMC_EV_SYSTEM] = c->mix_of[(e0batch[k] + (uint64_t)e) % c->mix_of.size()];
@@ -1983,8 +1988,7 @@ smc_status smc_run_graph(smc_ctx* c, uint64_t seed, uint64_t event0, int nev, do
     }
     c->have_moments = 1;
     if (ev_out) {
-      HIPCHK(hipMemcpyAsync(ev_out, c->evout, (size_t)nev * SMC_EV_STRIDE * sizeof(double),
-                            hipMemcpyDeviceToHost, c->stream));
+      to_host(c, ev_out, c->evout, (size_t)nev * SMC_EV_STRIDE * sizeof(double));
       sync(c);
       tag_systems(c, ev_out, nev);
     }
@@ -2220,8 +2224,7 @@ smc_status smc_fetch_events(smc_ctx* c, int nev, double* ev_out) {
   if (!c || !ev_out) return SMC_ERR_ARG;
   try {
     if (!c->have_moments || nev > c->nev) throw SmcError(SMC_ERR_STATE, "no moments for these events");
-    HIPCHK(hipMemcpyAsync(ev_out, c->evout, (size_t)nev * SMC_EV_STRIDE * sizeof(double), hipMemcpyDeviceToHost,
-                          c->stream));
+    to_host(c, ev_out, c->evout, (size_t)nev * SMC_EV_STRIDE * sizeof(double));
     sync(c);
     tag_systems(c, ev_out, nev);
     return SMC_OK;

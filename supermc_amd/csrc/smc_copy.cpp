@@ -1,0 +1,113 @@
+// smc_copy.cpp -- pageable device-to-host copies by worker threads (smc_copy.h)
+#include "smc_copy.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace smc {
+
+namespace {
+
+int workers_for(size_t pieces) {
+  const int hc = (int)std::thread::hardware_concurrency();
+  return (int)std::min<size_t>(pieces, (size_t)std::max(1, std::min(HostCopier::kWorkers, hc / 2)));
+}
+
+// f(0) .. f(n - 1) at once, f(0) on this thread; where a thread cannot be
+// started, on this one
+template <class F>
+void run_workers(int n, const F& f) {
+  std::vector<std::thread> th;
+  std::vector<int> left;
+  th.reserve(n);
+  left.reserve(n);
+  for (int i = 1; i < n; ++i) {
+    try {
+      th.emplace_back(f, i);
+    } catch (const std::system_error&) {
+      left.push_back(i);
+    }
+  }
+  f(0);
+  for (int i : left) f(i);
+  for (auto& t : th) t.join();
+}
+
+}  // namespace
+
+HostCopier::~HostCopier() {
+  for (int i = 0; i < kWorkers; ++i) {
+    if (done_[i]) (void)hipEventDestroy(done_[i]);
+    if (slot_[i]) (void)hipHostFree(slot_[i]);
+  }
+}
+
+bool HostCopier::staged(const void* dst, size_t bytes) {
+  if (bytes < kStagedBytes) return false;
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, dst) != hipSuccess) {
+    (void)hipGetLastError();  // memory the runtime does not know: pageable
+    return true;
+  }
+  return at.type == hipMemoryTypeUnregistered;
+}
+
+hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+  if (!staged(dst, bytes)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+  const size_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
+  const int n = workers_for(pieces);
+  int dev = 0;
+  hipError_t rc = hipGetDevice(&dev);
+  for (int i = 0; i < n && rc == hipSuccess; ++i) {
+    if (!slot_[i]) rc = hipHostMalloc(&slot_[i], kSlotBytes, hipHostMallocDefault);
+    if (rc == hipSuccess && !done_[i]) rc = hipEventCreateWithFlags(&done_[i], hipEventDisableTiming);
+  }
+  if (rc != hipSuccess) return rc;
+  std::atomic<size_t> next{0};
+  std::atomic<int> err{(int)hipSuccess};
+  std::mutex order;  // pieces are queued in the order they are taken
+  const auto work = [&](int i) {
+    if (hipSetDevice(dev) != hipSuccess) {
+      err = (int)hipErrorInvalidDevice;
+      return;
+    }
+    while (err.load() == (int)hipSuccess) {
+      size_t off, m;
+      hipError_t e;
+      {
+        const std::lock_guard<std::mutex> g(order);
+        const size_t p = next++;
+        if (p >= pieces) return;
+        off = p * kSlotBytes;
+        m = std::min(kSlotBytes, bytes - off);
+        e = hipMemcpyAsync(slot_[i], (const char*)src + off, m, hipMemcpyDeviceToHost, stream);
+        if (e == hipSuccess) e = hipEventRecord(done_[i], stream);
+      }
+      if (e == hipSuccess) e = hipEventSynchronize(done_[i]);
+      if (e != hipSuccess) {
+        err = (int)e;
+        return;
+      }
+      std::memcpy((char*)dst + off, slot_[i], m);
+    }
+  };
+  run_workers(n, work);
+  return (hipError_t)err.load();
+}
+
+void parallel_memcpy(void* dst, const void* src, size_t bytes) {
+  constexpr size_t kPiece = (size_t)1 << 20;
+  const int n = bytes < (size_t)4 << 20 ? 1 : workers_for(bytes / kPiece);
+  const size_t per = (bytes / n + 4095) & ~(size_t)4095;
+  run_workers(n, [&](int i) {
+    const size_t off = std::min(bytes, per * i), m = std::min(per, bytes - off);
+    if (m) std::memcpy((char*)dst + off, (const char*)src + off, m);
+  });
+}
+
+}  // namespace smc

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/smc_p3d.h"
+#include "smc_copy.h"
 #include "smc_internal.h"
 
 using namespace smc;
@@ -21,7 +22,15 @@ struct smc_p3d {
   double* tab = nullptr;                // device: eta, proj, targ
   hipStream_t stream = nullptr;
   std::string err;
+  // kept from call to call, grown as needed: source lists, and a grid buffer
+  // of at most kP3dGridBytes (one event's grid if that is larger)
+  char* lists = nullptr;
+  size_t lists_bytes = 0, lists_used = 0;
+  float* grid = nullptr;
+  size_t grid_floats = 0;
+  HostCopier copier;
 };
+constexpr size_t kP3dGridBytes = (size_t)256 << 20;
 
 namespace {
 
@@ -41,20 +50,31 @@ smc_status p3d_fail(smc_p3d* h, const P3dError& e) {
   return e.code;
 }
 
-// device buffer freed at scope exit
+constexpr size_t kAlign = 256;
 template <typename T>
-struct DevBuf {
-  T* p = nullptr;
-  explicit DevBuf(size_t n) {
-    if (n == 0) n = 1;
-    P3D_HIP(hipMalloc(&p, n * sizeof(T)));
-  }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-};
+size_t list_bytes(size_t n) {
+  return (n * sizeof(T) + kAlign - 1) / kAlign * kAlign;
+}
+
+// Room for bytes of lists in h's buffer, from its start.  Every call that
+// used the buffer has waited for its work.
+void reserve_lists(smc_p3d* h, size_t bytes) {
+  h->lists_used = 0;
+  if (h->lists_bytes >= bytes) return;
+  if (h->lists) (void)hipFree(h->lists);
+  h->lists = nullptr;
+  h->lists_bytes = 0;
+  P3D_HIP(hipMalloc(&h->lists, bytes));
+  h->lists_bytes = bytes;
+}
+
+template <typename T>
+T* take(smc_p3d* h, size_t n) {
+  T* p = reinterpret_cast<T*>(h->lists + h->lists_used);
+  h->lists_used += list_bytes<T>(n);
+  if (h->lists_used > h->lists_bytes) throw P3dError(SMC_ERR_CAPACITY, "list buffer too small");
+  return p;
+}
 
 template <typename T>
 void upload(T* dst, const T* src, size_t n, hipStream_t s) {
@@ -98,26 +118,64 @@ size_t grid_cells(const smc_p3d* h) {
   return (size_t)h->p.grid_neta * h->p.grid_nx * h->p.grid_ny;
 }
 
-void sample_dev(smc_p3d* h, int nev, const double* part_xy, const int* part_id, const int* part_off,
-                const double* bin_xy, const int* bin_off, uint64_t seed, uint64_t event0, double* d_psrc,
-                double* d_bsrc, int* d_poff, int* d_boff) {
-  const int np = check_offsets(part_off, nev, "participants");
-  const int nb = check_offsets(bin_off, nev, "binary collisions");
+// The source records of both lists on the device.
+struct Sources {
+  double *part, *bin;       // records, 6 doubles each
+  int *part_off, *bin_off;  // [nev + 1]
+  int np, nb;
+};
+
+Sources sample_dev(smc_p3d* h, int nev, const double* part_xy, const int* part_id, const int* part_off,
+                   const double* bin_xy, const int* bin_off, uint64_t seed, uint64_t event0) {
+  Sources s{};
+  s.np = check_offsets(part_off, nev, "participants");
+  s.nb = check_offsets(bin_off, nev, "binary collisions");
+  const size_t np = (size_t)s.np, nb = (size_t)s.nb;
   if ((np && (!part_xy || !part_id)) || (nb && !bin_xy)) throw P3dError(SMC_ERR_ARG, "source arrays missing");
-  DevBuf<double> pxy(2 * (size_t)np), bxy(2 * (size_t)nb);
-  DevBuf<int> pid(np), st(1);
-  upload(pxy.p, part_xy, 2 * (size_t)np, h->stream);
-  upload(bxy.p, bin_xy, 2 * (size_t)nb, h->stream);
-  upload(pid.p, part_id, (size_t)np, h->stream);
-  upload(d_poff, part_off, (size_t)nev + 1, h->stream);
-  upload(d_boff, bin_off, (size_t)nev + 1, h->stream);
-  P3D_HIP(hipMemsetAsync(st.p, 0, sizeof(int), h->stream));
-  P3D_HIP((hipError_t)launch_p3d_sample(cfg_of(h), seed, event0, nev, pxy.p, pid.p, d_poff, bxy.p, d_boff, d_psrc,
-                                        d_bsrc, st.p, h->stream));
+  reserve_lists(h, list_bytes<double>(8 * np) + list_bytes<double>(8 * nb) + 2 * list_bytes<int>((size_t)nev + 1) +
+                       list_bytes<int>(np) + list_bytes<int>(1) + 4 * kAlign);
+  s.part = take<double>(h, 6 * np);
+  s.bin = take<double>(h, 6 * nb);
+  s.part_off = take<int>(h, (size_t)nev + 1);
+  s.bin_off = take<int>(h, (size_t)nev + 1);
+  double *pxy = take<double>(h, 2 * np), *bxy = take<double>(h, 2 * nb);
+  int *pid = take<int>(h, np), *st = take<int>(h, 1);
+  upload(pxy, part_xy, 2 * np, h->stream);
+  upload(bxy, bin_xy, 2 * nb, h->stream);
+  upload(pid, part_id, np, h->stream);
+  upload(s.part_off, part_off, (size_t)nev + 1, h->stream);
+  upload(s.bin_off, bin_off, (size_t)nev + 1, h->stream);
+  P3D_HIP(hipMemsetAsync(st, 0, sizeof(int), h->stream));
+  P3D_HIP((hipError_t)launch_p3d_sample(cfg_of(h), seed, event0, nev, pxy, pid, s.part_off, bxy, s.bin_off, s.part,
+                                        s.bin, st, h->stream));
   int status = 0;
-  P3D_HIP(hipMemcpyAsync(&status, st.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  P3D_HIP(hipMemcpyAsync(&status, st, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   P3D_HIP(hipStreamSynchronize(h->stream));
   if (status) throw P3dError(SMC_ERR_ARG, "eta sampling did not accept within 65536 draws");
+  return s;
+}
+
+// Grids of nev events of one source list to host memory, through the grid
+// buffer a few events at a time.  On one stream: the smearing is a twentieth
+// of the copy, and a second stream for the copies made a call 2.7 times
+// slower whenever the runtime gave both streams one hardware queue.
+void grids_to_host(smc_p3d* h, int nev, const double* src, const int* off, float* out) {
+  const P3dCfg c = cfg_of(h);
+  const size_t cells = grid_cells(h);
+  const int per = (int)std::min<size_t>((size_t)nev, std::max<size_t>(1, kP3dGridBytes / (cells * sizeof(float))));
+  if (h->grid_floats < per * cells) {
+    if (h->grid) (void)hipFree(h->grid);
+    h->grid = nullptr;
+    h->grid_floats = 0;
+    P3D_HIP(hipMalloc(&h->grid, per * cells * sizeof(float)));
+    h->grid_floats = per * cells;
+  }
+  for (int e = 0; e < nev; e += per) {
+    const int n = std::min(per, nev - e);
+    P3D_HIP((hipError_t)launch_p3d_smear(c, n, src, off + e, h->grid, h->stream));
+    P3D_HIP(h->copier.copy(out + (size_t)e * cells, h->grid, (size_t)n * cells * sizeof(float), h->stream));
+  }
+  P3D_HIP(hipStreamSynchronize(h->stream));
 }
 
 }  // namespace
@@ -183,6 +241,8 @@ smc_status smc_p3d_create(smc_p3d** out, const smc_p3d_params* p) {
 void smc_p3d_destroy(smc_p3d* h) {
   if (!h) return;
   if (h->tab) (void)hipFree(h->tab);
+  if (h->lists) (void)hipFree(h->lists);
+  if (h->grid) (void)hipFree(h->grid);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -204,14 +264,11 @@ smc_status smc_p3d_sample(smc_p3d* h, int nev, const double* part_xy, const int*
   if (!h || nev < 0) return SMC_ERR_ARG;
   if (nev == 0) return SMC_OK;
   try {
-    const int np = check_offsets(part_off, nev, "participants"), nb = check_offsets(bin_off, nev, "binary collisions");
-    DevBuf<double> ps(6 * (size_t)np), bs(6 * (size_t)nb);
-    DevBuf<int> po((size_t)nev + 1), bo((size_t)nev + 1);
-    sample_dev(h, nev, part_xy, part_id, part_off, bin_xy, bin_off, seed, event0, ps.p, bs.p, po.p, bo.p);
-    if (part_src && np)
-      P3D_HIP(hipMemcpyAsync(part_src, ps.p, 6 * (size_t)np * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    if (bin_src && nb)
-      P3D_HIP(hipMemcpyAsync(bin_src, bs.p, 6 * (size_t)nb * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    const Sources src = sample_dev(h, nev, part_xy, part_id, part_off, bin_xy, bin_off, seed, event0);
+    if (part_src && src.np)
+      P3D_HIP(hipMemcpyAsync(part_src, src.part, 6 * (size_t)src.np * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    if (bin_src && src.nb)
+      P3D_HIP(hipMemcpyAsync(bin_src, src.bin, 6 * (size_t)src.nb * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     P3D_HIP(hipStreamSynchronize(h->stream));
     return SMC_OK;
   } catch (const P3dError& e) { return p3d_fail(h, e); }
@@ -226,15 +283,12 @@ smc_status smc_p3d_smear(smc_p3d* h, int nev, const double* src, const int* src_
     for (int i = 0; i < n; ++i)
       if (!(src[6 * (size_t)i + 3] > 0 && src[6 * (size_t)i + 4] > 0 && src[6 * (size_t)i + 5] > 0))
         throw P3dError(SMC_ERR_ARG, "source widths must be positive");
-    DevBuf<double> s(6 * (size_t)n);
-    DevBuf<int> off((size_t)nev + 1);
-    const size_t cells = grid_cells(h) * nev;
-    DevBuf<float> g(cells);
-    upload(s.p, src, 6 * (size_t)n, h->stream);
-    upload(off.p, src_off, (size_t)nev + 1, h->stream);
-    P3D_HIP((hipError_t)launch_p3d_smear(cfg_of(h), nev, s.p, off.p, g.p, h->stream));
-    P3D_HIP(hipMemcpyAsync(rho, g.p, cells * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-    P3D_HIP(hipStreamSynchronize(h->stream));
+    reserve_lists(h, list_bytes<double>(6 * (size_t)n) + list_bytes<int>((size_t)nev + 1) + 2 * kAlign);
+    double* s = take<double>(h, 6 * (size_t)n);
+    int* off = take<int>(h, (size_t)nev + 1);
+    upload(s, src, 6 * (size_t)n, h->stream);
+    upload(off, src_off, (size_t)nev + 1, h->stream);
+    grids_to_host(h, nev, s, off, rho);
     return SMC_OK;
   } catch (const P3dError& e) { return p3d_fail(h, e); }
 }
@@ -245,28 +299,13 @@ smc_status smc_p3d_generate(smc_p3d* h, int nev, const double* part_xy, const in
   if (!h || nev < 0) return SMC_ERR_ARG;
   if (nev == 0) return SMC_OK;
   try {
-    const int np = check_offsets(part_off, nev, "participants"), nb = check_offsets(bin_off, nev, "binary collisions");
-    DevBuf<double> ps(6 * (size_t)np), bs(6 * (size_t)nb);
-    DevBuf<int> po((size_t)nev + 1), bo((size_t)nev + 1);
-    sample_dev(h, nev, part_xy, part_id, part_off, bin_xy, bin_off, seed, event0, ps.p, bs.p, po.p, bo.p);
-    const size_t cells = grid_cells(h) * nev;
-    const P3dCfg c = cfg_of(h);
-    if (rho_part) {
-      DevBuf<float> g(cells);
-      P3D_HIP((hipError_t)launch_p3d_smear(c, nev, ps.p, po.p, g.p, h->stream));
-      P3D_HIP(hipMemcpyAsync(rho_part, g.p, cells * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-      P3D_HIP(hipStreamSynchronize(h->stream));
-    }
-    if (rho_binary) {
-      DevBuf<float> g(cells);
-      P3D_HIP((hipError_t)launch_p3d_smear(c, nev, bs.p, bo.p, g.p, h->stream));
-      P3D_HIP(hipMemcpyAsync(rho_binary, g.p, cells * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-      P3D_HIP(hipStreamSynchronize(h->stream));
-    }
-    if (part_src && np)
-      P3D_HIP(hipMemcpyAsync(part_src, ps.p, 6 * (size_t)np * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    if (bin_src && nb)
-      P3D_HIP(hipMemcpyAsync(bin_src, bs.p, 6 * (size_t)nb * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    const Sources src = sample_dev(h, nev, part_xy, part_id, part_off, bin_xy, bin_off, seed, event0);
+    if (rho_part) grids_to_host(h, nev, src.part, src.part_off, rho_part);
+    if (rho_binary) grids_to_host(h, nev, src.bin, src.bin_off, rho_binary);
+    if (part_src && src.np)
+      P3D_HIP(hipMemcpyAsync(part_src, src.part, 6 * (size_t)src.np * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    if (bin_src && src.nb)
+      P3D_HIP(hipMemcpyAsync(bin_src, src.bin, 6 * (size_t)src.nb * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     P3D_HIP(hipStreamSynchronize(h->stream));
     return SMC_OK;
   } catch (const P3dError& e) { return p3d_fail(h, e); }
