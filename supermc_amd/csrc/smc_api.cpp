@@ -595,6 +595,7 @@ void alloc_buffers(smc_ctx* c) {
   b.counts = dalloc<int>(E * 8);
   b.bval = dalloc<double>(E);
   b.order = dalloc<int>(E);
+  b.evkey = dalloc<uint4>(E);
   b.raw = dalloc<int>(E * 2 * kAMax * 2);
   b.src_cap = 2 * kAMax + (int)MP;
   b.src = dalloc<int4>(E * (size_t)b.src_cap);
@@ -1378,7 +1379,7 @@ void smc_destroy(smc_ctx* c) {
   if (c->d_mix_of) (void)hipFree(c->d_mix_of);
   for (auto& pe : c->pending) { (void)hipEventDestroy(pe.a); (void)hipEventDestroy(pe.b); }
   void* ptrs[] = {c->buf.pos, c->buf.fluct, c->buf.wound, c->buf.pairs, c->buf.pfluct, c->buf.paw, c->buf.counts,
-                  c->buf.bval, c->buf.order, c->buf.raw, c->buf.src, c->buf.swin, c->dtab, c->grid, c->ta, c->tb, c->tmp, c->evout,
+                  c->buf.bval, c->buf.evkey, c->buf.order, c->buf.raw, c->buf.src, c->buf.swin, c->dtab, c->grid, c->ta, c->tb, c->tmp, c->evout,
                   c->cm, c->band, c->mrects, c->nmrect, c->avg_rot, c->avg_acc, c->avg_sum, c->avg_part, c->avg_ext, c->aux0,
                   c->aux1, c->grid64, c->spec_src, c->spec_swin, c->spec_counts, c->kln_table, c->kln_ptf, c->kln_nodes_f, c->kln_ptd, c->kln_nodes_d, c->kln_list,
                   c->kln_breaks.bu, c->kln_breaks.bv, c->kln_breaks.sorted, c->kln_breaks.tab};

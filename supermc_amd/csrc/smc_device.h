@@ -14,8 +14,9 @@ namespace smc {
 __device__ __forceinline__ uint4 philox(uint4 c, uint2 k) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    const unsigned lo0 = 0xD2511F53u * c.x, hi0 = __umulhi(0xD2511F53u, c.x);
-    const unsigned lo1 = 0xCD9E8D57u * c.z, hi1 = __umulhi(0xCD9E8D57u, c.z);
+    // both halves of a product from one multiply-add (v_mad_u64_u32)
+    const unsigned long long p0 = (unsigned long long)0xD2511F53u * c.x, p1 = (unsigned long long)0xCD9E8D57u * c.z;
+    const unsigned lo0 = (unsigned)p0, hi0 = (unsigned)(p0 >> 32), lo1 = (unsigned)p1, hi1 = (unsigned)(p1 >> 32);
     c = make_uint4(hi1 ^ c.y ^ k.x, lo1, hi0 ^ c.w ^ k.y, lo0);
     k.x += 0x9E3779B9u;
     k.y += 0xBB67AE85u;
@@ -67,6 +68,27 @@ __device__ __forceinline__ int step_eval(const StepTable& T, int p) {
   while (k < T.n && T.thr[k] <= p) ++k;
   while (k > 0 && T.thr[k - 1] > p) --k;
   return T.vlo + k;
+}
+
+// The low and high edges (tables lo and hi) of a window at p: both tables'
+// guesses and the thresholds around them are read before either is used.
+__device__ __forceinline__ int step_window(const StepTable& lo, const StepTable& hi, int p) {
+  int k[2];
+  const StepTable* const T[2] = {&lo, &hi};
+  bool ok = true;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const StepTable& t = *T[i];
+    if (t.n == 0) {
+      k[i] = 0;
+      continue;
+    }
+    k[i] = max(0, min(t.n, (int)floorf(fmaf(t.a, (float)p, t.b))));
+    const int below = t.thr[max(k[i] - 1, 0)], above = t.thr[min(k[i], t.n - 1)];
+    ok = ok && (k[i] == 0 || below <= p) && (k[i] == t.n || above > p);
+  }
+  if (!ok) return step_eval(lo, p) | (step_eval(hi, p) << 16);
+  return (lo.vlo + k[0]) | ((hi.vlo + k[1]) << 16);
 }
 
 __device__ __forceinline__ int quant(float v) { return (int)rintf(v * 16777216.0f); }
@@ -209,56 +231,15 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// 256-thread exclusive scan through LDS (tmp has 256 ints).
-__device__ inline int block_excl_scan(int v, int* tmp) {
-  const int t = threadIdx.x;
-  tmp[t] = v;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const int add = (t >= off) ? tmp[t - off] : 0;
-    __syncthreads();
-    tmp[t] += add;
-    __syncthreads();
-  }
-  const int incl = tmp[t];
-  __syncthreads();
-  return incl - v;
-}
-
-// Ascending bitonic sort of key[0][0..255] and key[1][0..255] by a
-// 256-thread workgroup (threads 0-127 sort key[0], 128-255 key[1]); ends
-// with a barrier.
-__device__ inline void bitonic_sort_2x256(unsigned long long (*key)[256]) {
-  const int t = threadIdx.x, a = t >> 7, p = t & 127;
-  __syncthreads();
-  for (int k = 2; k <= 256; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const int i = ((p & ~(j - 1)) << 1) | (p & (j - 1));
-      const int l = i + j;
-      const bool up = (i & k) == 0;
-      const unsigned long long x = key[a][i], y = key[a][l];
-      if ((x > y) == up) {
-        key[a][i] = y;
-        key[a][l] = x;
-      }
-      __syncthreads();
-    }
-}
-
 // Exact footprints of a source at (ph, qh) half quanta: the participant box
 // (MCnucl.cpp:831-844) and the +-5w window (MCnucl.cpp:450-457, 729-736),
 // each packed as lo | hi << 16 per axis.
 __device__ __forceinline__ int4 src_windows(const DevCfg& cfg, int ph, int qh, bool box) {
   int4 w;
-  if (box) {
-    w.x = step_eval(cfg.tab[kBoxLoX], ph) | (step_eval(cfg.tab[kBoxHiX], ph) << 16);
-    w.y = step_eval(cfg.tab[kBoxLoY], qh) | (step_eval(cfg.tab[kBoxHiY], qh) << 16);
-  } else {
-    w.x = 0;
-    w.y = 0;
-  }
-  w.z = step_eval(cfg.tab[kWinLoX], ph) | (step_eval(cfg.tab[kWinHiX], ph) << 16);
-  w.w = step_eval(cfg.tab[kWinLoY], qh) | (step_eval(cfg.tab[kWinHiY], qh) << 16);
+  w.x = box ? step_window(cfg.tab[kBoxLoX], cfg.tab[kBoxHiX], ph) : 0;
+  w.y = box ? step_window(cfg.tab[kBoxLoY], cfg.tab[kBoxHiY], qh) : 0;
+  w.z = step_window(cfg.tab[kWinLoX], cfg.tab[kWinHiX], ph);
+  w.w = step_window(cfg.tab[kWinLoY], cfg.tab[kWinHiY], qh);
   return w;
 }
 

@@ -106,6 +106,7 @@ struct EvBufs {
   int* counts;     // [ev][8]: npartA, npartB, ncoll, status, attempts, nsrc,
                    //   source rectangle x0 | x1 << 16, y0 | y1 << 16 (cells)
   double* bval;    // [ev]
+  uint4* evkey;    // [ev] {seed lo, hi, event index lo, hi} of the event's draws
   int* raw;        // [ev][2][kAMax][2] fed positions (quanta), input order
   int4* src;       // [ev][src_cap] {x_h, y_h, fluct bits, kind}
   int4* swin;      // [ev][src_cap] footprints {box x, box y, 5w x, 5w y}, lo | hi << 16

@@ -442,3 +442,46 @@ def test_rectangular_grid_and_cells_match_oracle(path, model):
             _check_event_record(rec[e], o, p)
             checked += 1
         assert checked >= 3
+
+
+@pytest.mark.parametrize("layout", ["one column", "one row", "lattice", "far", "mirrored"])
+@pytest.mark.parametrize("sizes", [(208, 208), (1, 208), (64, 65), (238, 5)])
+def test_collision_order_with_equal_and_crowded_positions(layout, sizes):
+    """The sort by x and the wound order where they have most to decide: all
+    nucleons at one x (one bin, ties by input index), all in one row, on a
+    coarse lattice (many equal x), beyond the bins' +-16 fm on both sides, and
+    both nuclei with the same positions in opposite input order.  Pair lists,
+    participants and wound order equal the oracle's."""
+    from supermc_amd import Context
+    rng = np.random.default_rng(sum(sizes))
+    A, B = sizes
+
+    def nucleus(n):
+        y = rng.uniform(-4, 4, n)
+        x = {"one column": np.full(n, 0.375), "one row": rng.uniform(-4, 4, n),
+             "lattice": rng.integers(-6, 7, n) * 0.5, "far": rng.choice([-21.0, 21.0], n) + rng.uniform(-5, 5, n),
+             "mirrored": rng.uniform(-3, 3, n)}[layout]
+        if layout == "one row":
+            y = np.full(n, 0.25)
+        return np.round(np.stack([x, y], -1) / H.Q) * H.Q
+
+    xa, xb = nucleus(A), nucleus(B)
+    if layout == "mirrored":
+        xb = np.resize(xa[::-1], (B, 2)).copy()
+    p = H.glauber_params("PbPb", Aproj=A, Atarg=B, max_events=1, cc_fluctuation_model=0, max_pairs=A * B)
+    with Context(p) as ctx:
+        ctx.set_positions(xa[None], xb[None])
+        o = H.oracle_event(ctx, 0)
+        pa, pb, _ = o["gpu_pairs"]
+        assert np.array_equal(pa, o["col"]["pair_a"]) and np.array_equal(pb, o["col"]["pair_b"])
+        na, nb, nc, _ = ctx.collide(allow=(4,))
+        assert (na[0], nb[0], nc[0]) == (o["col"]["npart_a"], o["col"]["npart_b"], len(pa))
+        # input indices in collision order: by x, equal x by input index
+        for side, x in (("proj", xa), ("targ", xb)):
+            assert np.array_equal(o["nuc"]["xy_" + side], x[np.lexsort((np.arange(len(x)), x[:, 0]))])
+        # wound order: projectile rows as sorted, targets by first hitting row, then index
+        wa, wb = o["nuc"]["wound_proj"], o["nuc"]["wound_targ"]
+        assert np.array_equal(np.flatnonzero(wa >= 0), np.unique(pa)) and np.array_equal(wa[wa >= 0], np.arange(na[0]))
+        first = {j: i for i, j in reversed(list(zip(pa, pb)))}
+        order = sorted(first, key=lambda j: (first[j], j))
+        assert [int(wb[j]) for j in order] == list(range(len(order))) and (wb >= 0).sum() == len(order)
