@@ -170,6 +170,7 @@ __device__ void build_mask(const DevCfg& cfg, const EvBufs& buf, int e, unsigned
   {
     const int offx = step_eval(cfg.tab[kOffX], rxl), offy = step_eval(cfg.tab[kOffY], ryl);
     const unsigned long long m = __ballot(part);
+    __syncthreads();  // every wave has read the box edges
     if (lane == 0) L.ired[wv][0] = __popcll(m);
     __syncthreads();
     int base = 0, np = 0;
