@@ -1145,14 +1145,15 @@ void diff_setup(smc_ctx* c, uint64_t seed, uint64_t event0, int nev) {
   d.gev = dif_alloc<double>(c, 11, E * 5);
   d.wstab = dif_alloc<double>(c, 13, kWsTabLen);
   d.cotc = dif_alloc<double>(c, 14, E * kCotStride);
-  std::vector<double> x, w;
-  gauss_legendre01(64, x, w);
-  std::vector<double> glh(128);
-  for (int i = 0; i < 64; ++i) {
-    glh[2 * i] = x[i];
-    glh[2 * i + 1] = w[i];
+  std::vector<double> x, w, glh;
+  for (int n : {64, kWsNear}) {
+    gauss_legendre01(n, x, w);
+    for (int i = 0; i < n; ++i) {
+      glh.push_back(x[i]);
+      glh.push_back(w[i]);
+    }
   }
-  double* gl = dif_alloc<double>(c, 12, 128);
+  double* gl = dif_alloc<double>(c, 12, glh.size());
   HIPCHK(hipMemcpy(gl, glh.data(), glh.size() * sizeof(double), hipMemcpyHostToDevice));
   d.gl = reinterpret_cast<const double2*>(gl);
   d.ngl = 64;

@@ -30,18 +30,26 @@ struct WsInt {
   double n, nR, na;
 };
 
+__device__ __forceinline__ void ws_add(WsInt& s, double t, double wt, double R, double a) {
+  const double rho = 1.0 / (1.0 + exp((t - R) / a));
+  const double dR = rho * (1.0 - rho) / a;
+  const double t2w = t * t * wt;
+  s.n += t2w * rho;
+  s.nR += t2w * dR;
+  s.na += t2w * dR * (t - R) / a;
+}
+
 __device__ inline WsInt ws_integrals(double r, double R, double a, const double2* gl, int ngl) {
   WsInt s{0.0, 0.0, 0.0};
-  for (int j = 0; j < ngl; ++j) {
-    const double t = r * gl[j].x, wt = r * gl[j].y;
-    const double rho = 1.0 / (1.0 + exp((t - R) / a));
-    const double dR = rho * (1.0 - rho) / a;
-    const double t2w = t * t * wt;
-    s.n += t2w * rho;
-    s.nR += t2w * dR;
-    s.na += t2w * dR * (t - R) / a;
-  }
+  for (int j = 0; j < ngl; ++j) ws_add(s, r * gl[j].x, r * gl[j].y, R, a);
   return s;
+}
+
+// the same by a wavefront, one node per lane
+__device__ inline WsInt ws_integrals_wave(double r, double R, double a, const double2* gl, int ngl) {
+  WsInt s{0.0, 0.0, 0.0};
+  for (int j = threadIdx.x & 63; j < ngl; j += 64) ws_add(s, r * gl[j].x, r * gl[j].y, R, a);
+  return WsInt{wave_sum(s.n), wave_sum(s.nR), wave_sum(s.na)};
 }
 
 // Normalisation Z = N(R + 2.5) and its R and a derivatives (the upper limit
@@ -49,42 +57,28 @@ __device__ inline WsInt ws_integrals(double r, double R, double a, const double2
 struct WsNorm {
   double n, R, a;
 };
-__device__ inline WsNorm ws_norm(double R, double a, const double2* gl, int ngl) {
+__device__ inline WsNorm ws_norm_wave(double R, double a, const double2* gl, int ngl) {
   const double rmax = R + 2.5;
-  const WsInt Z = ws_integrals(rmax, R, a, gl, ngl);
+  const WsInt Z = ws_integrals_wave(rmax, R, a, gl, ngl);
   const double rhomax = 1.0 / (1.0 + exp(2.5 / a));
   return WsNorm{Z.n, Z.nR + rmax * rmax * rhomax, Z.na};
 }
 
-// r = F^{-1}(u; R, a) on [0, R + 2.5] and dr/dR, dr/da.  tab (optional):
-// kWsTab quantiles r at v = u^(1/3) = i/(kWsTab-1) for this (R, a), then
-// {Z, Z_R, Z_a} (k_ws_table).  With it, Newton starts from the cubic
-// interpolation of the table (error ~1e-12 fm) and usually stops after one
-// step.  Newton stops once a step is below 1e-9 (R + 2.5): in the quadratic
-// regime the root is then within ~1e-16 fm of the new point.  The R and a
-// derivatives come from the last evaluation, within that step of r.
-__device__ inline void ws_finv(double u, double R, double a, const double2* gl, int ngl, double& r, double& rR,
-                               double& ra, const double* tab = nullptr) {
+// r = F^{-1}(u; R, a) on [0, R + 2.5] and dr/dR, dr/da by Newton's iteration
+// from x; integ(x) gives N(x) and its derivatives.  Newton stops once a step
+// is below 1e-9 (R + 2.5): in the quadratic regime the root is then within
+// ~1e-16 fm of the new point.  The R and a derivatives come from the last
+// evaluation, within that step of r.
+template <class Integ>
+__device__ inline void ws_newton(double u, double R, double a, const WsNorm& Z, double x, Integ integ, double& r,
+                                 double& rR, double& ra) {
   const double rmax = R + 2.5;
-  const WsNorm Z = tab ? WsNorm{tab[kWsTab], tab[kWsTab + 1], tab[kWsTab + 2]} : ws_norm(R, a, gl, ngl);
   const double target = u * Z.n;
-  double lo = 0.0, hi = rmax, x = rmax * cbrt(u);
-  if (tab) {
-    const double v = cbrt(u) * (kWsTab - 1);
-    const int i = min((int)v, kWsTab - 2);
-    const double f = v - i;
-    if (i >= 1 && i + 2 < kWsTab) {  // Lagrange cubic through nodes i-1 .. i+2
-      const double wm = -f * (f - 1.0) * (f - 2.0) / 6.0, w0 = (f + 1.0) * (f - 1.0) * (f - 2.0) / 2.0;
-      const double w1 = -(f + 1.0) * f * (f - 2.0) / 2.0, w2 = (f + 1.0) * f * (f - 1.0) / 6.0;
-      x = wm * tab[i - 1] + w0 * tab[i] + w1 * tab[i + 1] + w2 * tab[i + 2];
-    } else {
-      x = tab[i] + f * (tab[i + 1] - tab[i]);
-    }
-  }
+  double lo = 0.0, hi = rmax;
   WsInt N{0.0, 0.0, 0.0};
   double xe = x, rho = 0.0;  // last evaluation point and rho there
   for (int it = 0; it < 100; ++it) {
-    N = ws_integrals(x, R, a, gl, ngl);
+    N = integ(x);
     const double fv = N.n - target;
     if (fv < 0.0) lo = x;
     else hi = x;
@@ -104,6 +98,45 @@ __device__ inline void ws_finv(double u, double R, double a, const double2* gl, 
   const double Fa = N.na / Z.n - N.n * Z.a / (Z.n * Z.n);
   rR = -FR / Fr;
   ra = -Fa / Fr;
+}
+
+// The quantile from the table of this (R, a) (k_ws_table).  Newton starts
+// from the cubic interpolation of the table (error ~1e-12 fm) and usually
+// stops after one step.  N(x) is the nearest node's N plus the integral from
+// there, on kWsNear Gauss-Legendre nodes where the distance is at most a/2:
+// the integrand's poles lie pi a off the axis, so the rule's error there is
+// below 25^-12 of that part.  Farther away (the last cells of a small a) N
+// is integrated from 0 over all nodes, as the table's own entries are.  One
+// evaluation per nucleon takes 6 of its 64 exponentials: k_diff_pos
+// 0.91 -> 0.15 ms per 4096 Pb+Pb events.
+__device__ inline void ws_finv(double u, double R, double a, const double2* gl, int ngl, const double* tab, double& r,
+                               double& rR, double& ra) {
+  const WsNorm Z{tab[kWsTab], tab[kWsTab + 1], tab[kWsTab + 2]};
+  const double v = cbrt(u) * (kWsTab - 1);
+  const int i = min((int)v, kWsTab - 2);
+  const double f = v - i;
+  double x;
+  if (i >= 1 && i + 2 < kWsTab) {  // Lagrange cubic through nodes i-1 .. i+2
+    const double wm = -f * (f - 1.0) * (f - 2.0) / 6.0, w0 = (f + 1.0) * (f - 1.0) * (f - 2.0) / 2.0;
+    const double w1 = -(f + 1.0) * f * (f - 2.0) / 2.0, w2 = (f + 1.0) * f * (f - 1.0) / 6.0;
+    x = wm * tab[i - 1] + w0 * tab[i] + w1 * tab[i + 1] + w2 * tab[i + 2];
+  } else {
+    x = tab[i] + f * (tab[i + 1] - tab[i]);
+  }
+  const int k = f < 0.5 ? i : i + 1;
+  const double* node = tab + kWsTabInt + 3 * k;
+  const double r0 = tab[k], reach = 0.5 * a;
+  const double2* near = gl + ngl;
+  ws_newton(
+      u, R, a, Z, x,
+      [&](double t1) {
+        const double h = t1 - r0;
+        if (!(fabs(h) <= reach)) return ws_integrals(t1, R, a, gl, ngl);
+        WsInt s{node[0], node[1], node[2]};
+        for (int j = 0; j < kWsNear; ++j) ws_add(s, r0 + h * near[j].x, h * near[j].y, R, a);
+        return s;
+      },
+      r, rR, ra);
 }
 
 // digamma by upward recurrence to z >= 12 and the asymptotic series
@@ -185,21 +218,32 @@ __device__ __forceinline__ double diff_shape(int kind, double alpha, double kg) 
   return (kind == kSrcPair) ? (alpha + 1e-8) * kg : (1.0 - alpha + 1e-8) * 0.5 * kg;
 }
 
-// The radial quantile at v = u^(1/3) = i/(kWsTab-1), i < kWsTab; thread 0
-// also stores {Z, Z_R, Z_a} after the table.
+// One wavefront per table node i: the radial quantile r at
+// v = u^(1/3) = i/(kWsTab-1) into tab[i] and N, N_R, N_a at that r into
+// tab[kWsTabInt + 3 i ..]; {Z, Z_R, Z_a} after the quantiles.  A node's
+// integrals are a chain of 64 terms, four to six times over: with one lane
+// per term the kernel takes 14 us instead of 157.
 __global__ __launch_bounds__(256) void k_ws_table(double R, double a, const double2* gl, int ngl, double* tab) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (i >= kWsTab) return;
+  const WsNorm z = ws_norm_wave(R, a, gl, ngl);
+  const double v = (double)i / (kWsTab - 1);
+  double r = 0.0, rR, ra;
+  if (i > 0)
+    ws_newton(
+        v * v * v, R, a, z, (R + 2.5) * v, [&](double x) { return ws_integrals_wave(x, R, a, gl, ngl); }, r, rR, ra);
+  const WsInt N = ws_integrals_wave(r, R, a, gl, ngl);
+  if (lane != 0) return;
   if (i == 0) {
-    const WsNorm z = ws_norm(R, a, gl, ngl);
     tab[kWsTab] = z.n;
     tab[kWsTab + 1] = z.R;
     tab[kWsTab + 2] = z.a;
   }
-  const double v = (double)i / (kWsTab - 1);
-  double r, rR, ra;
-  ws_finv(v * v * v, R, a, gl, ngl, r, rR, ra);
   tab[i] = r;
+  double* node = tab + kWsTabInt + 3 * i;
+  node[0] = N.n;
+  node[1] = N.nR;
+  node[2] = N.na;
 }
 
 // ------------------------------------------------------------- topology
@@ -240,7 +284,7 @@ __global__ __launch_bounds__(64) void k_diff_topo(DevCfg cfg, EvBufs buf, DiffBu
       const double c = 2.0 * u53(r2.x, r2.y) - 1.0;
       const double ph = 2.0 * M_PI * u53(r2.z, r2.w);
       double r, rR, ra;
-      ws_finv(u, R0, a0, d.gl, d.ngl, r, rR, ra, d.wstab);
+      ws_finv(u, R0, a0, d.gl, d.ngl, d.wstab, r, rR, ra);
       const double st = sqrt(fmax(0.0, 1.0 - c * c));
       const double x = r * st * cos(ph), y = r * st * sin(ph), z = r * c;
       bool good = true;
@@ -313,7 +357,7 @@ __global__ __launch_bounds__(256) void k_diff_pos(DevCfg cfg, DiffBufs d, double
     if (t < A) {
       const double* du = d.du + (((size_t)e * 2 + nu) * kAMax + t) * 4;
       double r, rR, ra;
-      ws_finv(du[0], R, a, d.gl, d.ngl, r, rR, ra, d.wstab);
+      ws_finv(du[0], R, a, d.gl, d.ngl, d.wstab, r, rR, ra);
       const double st = sqrt(fmax(0.0, 1.0 - du[1] * du[1]));
       const double nx = st * cos(du[2]), ny = st * sin(du[2]);
       v[0] = r * nx;
@@ -679,7 +723,7 @@ __global__ __launch_bounds__(256) void k_diff_chain(DevCfg cfg, EvBufs buf, Diff
 int launch_diff_topo(const DevCfg& cfg, const EvBufs& b, const DiffBufs& d, int nev, unsigned long long seed,
                      unsigned long long event0, double R0, double a0, void* stream) {
   const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
-  hipLaunchKernelGGL(k_ws_table, dim3((kWsTab + 255) / 256), dim3(256), 0, (hipStream_t)stream, R0, a0, d.gl, d.ngl,
+  hipLaunchKernelGGL(k_ws_table, dim3((kWsTab + 3) / 4), dim3(256), 0, (hipStream_t)stream, R0, a0, d.gl, d.ngl,
                      d.wstab);
   hipLaunchKernelGGL(k_diff_topo, dim3(nev), dim3(64), 0, (hipStream_t)stream, cfg, b, d, key, event0, R0, a0);
   return (int)hipGetLastError();
@@ -689,7 +733,7 @@ int launch_diff_forward_pre(const DevCfg& cfg, const EvBufs& b, const DiffBufs& 
                             unsigned long long event0, const double* theta, int fluct, void* stream) {
   const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_ws_table, dim3((kWsTab + 255) / 256), dim3(256), 0, st, theta[1], theta[2], d.gl, d.ngl,
+  hipLaunchKernelGGL(k_ws_table, dim3((kWsTab + 3) / 4), dim3(256), 0, st, theta[1], theta[2], d.gl, d.ngl,
                      d.wstab);
   hipLaunchKernelGGL(k_diff_pos, dim3(nev), dim3(256), 0, st, cfg, d, theta[1], theta[2]);
   hipLaunchKernelGGL(k_diff_src, dim3(nev), dim3(256), 0, st, cfg, b, d, key, event0, theta[3], theta[4], fluct);

@@ -134,14 +134,16 @@ struct DiffBufs {
   unsigned* mask;     // [ev][nx][(ny+31)/32] hot-spot mask at theta0
   double4* gsrc;      // [ev][src_cap] dL/dW, dL/dx, dL/dy, dL/dw per source
   double* gev;        // [ev][5] dL/dtheta per event
-  const double2* gl;  // Gauss-Legendre nodes/weights on [0, 1]
+  const double2* gl;  // Gauss-Legendre nodes/weights on [0, 1]: ngl, then kWsNear of a short rule
   int ngl;
-  double* wstab;      // [kWsTabLen] radial quantiles of the current (R, a) (Newton starts), then Z, Z_R, Z_a
+  double* wstab;      // [kWsTabLen] radial quantiles of the current (R, a), Z, Z_R, Z_a, the quantiles' N, N_R, N_a
   double* cotc;       // [ev][kCotStride] coefficients of the cell cotangents (k_diff_cot_coef)
 };
 constexpr int kCotStride = 12;  // c0, then (lam cx/S, lam cy/S, lam Ar/(Am N), lam Ai/(Am N), lam Am/N^2) for n = 2, 3
 constexpr int kWsTab = 2049;              // radial quantile nodes, uniform in u^(1/3)
-constexpr int kWsTabLen = kWsTab + 3;     // + the normalisation and its R, a derivatives
+constexpr int kWsTabInt = kWsTab + 3;     // + the normalisation and its R, a derivatives
+constexpr int kWsTabLen = kWsTabInt + 3 * kWsTab;  // + N and its R, a derivatives at the nodes
+constexpr int kWsNear = 6;                // nodes of the integral from the nearest table node
 // per-event scalars of the differentiable moments
 enum : int {
   kDsS = 0, kDsXc, kDsYc, kDsA2r, kDsA2i, kDsA3r, kDsA3i, kDsN, kDsMx, kDsMy,
