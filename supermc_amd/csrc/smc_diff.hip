@@ -176,27 +176,27 @@ __device__ inline double gamma_p(double s, double x, double lg1, double psi1, do
   return P;
 }
 
-// Unit-scale Gamma quantile x(v; s) (P(s, x) = v) and dx/ds.  Halley's
-// iteration (P' = pdf, P'' = pdf ((s-1)/x - 1)) from the small-x form
-// x0 = (v Gamma(s+1))^(1/s), which lies left of the root for every s > 0
-// (e^-x sum_n x^n / ((s+1)...(s+n)) < 1).  The bracket [lo, hi] is built
+// What a quantile needs of its shape alone.
+struct GammaShape {
+  double lg1, psi1, lgs;  // ln Gamma(s+1), psi(s+1), ln Gamma(s)
+};
+__device__ inline GammaShape gamma_shape(double s) {
+  const double lg1 = lgamma(s + 1.0);
+  return GammaShape{lg1, digamma_d(s + 1.0), lg1 - log(s)};
+}
+
+// Unit-scale Gamma quantile x(v; s) (P(s, x) = v).  Halley's iteration
+// (P' = pdf, P'' = pdf ((s-1)/x - 1)) from xx.  The bracket [lo, hi] is built
 // from the evaluations; a step that leaves it bisects (or doubles while hi
 // is open).  A Halley step below 1e-5 x leaves an error ~1e-15 x, so the
-// iteration stops there: about 3-4 evaluations of P per quantile.
-__device__ inline void gamma_qf(double v, double s, double& x, double& dxds) {
-  if (!(v > 0.0)) {
-    x = 0.0;
-    dxds = 0.0;
-    return;
-  }
-  const double lg1 = lgamma(s + 1.0), psi1 = digamma_d(s + 1.0), lgs = lg1 - log(s);
+// iteration stops there.
+__device__ inline double gamma_q(double v, double s, const GammaShape& g, double xx) {
   double lo = 0.0, hi = HUGE_VAL;
-  double xx = exp((log(v) + lg1) / s);
   for (int it = 0; it < 200; ++it) {
-    const double f = gamma_p(s, xx, lg1, psi1, nullptr) - v;
+    const double f = gamma_p(s, xx, g.lg1, g.psi1, nullptr) - v;
     if (f < 0.0) lo = xx;
     else hi = xx;
-    const double pdf = exp(-xx + (s - 1.0) * log(xx) - lgs);
+    const double pdf = exp(-xx + (s - 1.0) * log(xx) - g.lgs);
     const double d2 = pdf * ((s - 1.0) / xx - 1.0);
     const double den = 2.0 * pdf * pdf - f * d2;
     double xn = (den > 0.0) ? xx - 2.0 * f * pdf / den : xx - f / pdf;
@@ -206,10 +206,44 @@ __device__ inline void gamma_qf(double v, double s, double& x, double& dxds) {
     xx = xn;
     if (done) break;
   }
-  x = xx;
+  return xx;
+}
+
+// The small-x form (v Gamma(s+1))^(1/s), which lies left of the root for
+// every s > 0 (e^-x sum_n x^n / ((s+1)...(s+n)) < 1).
+__device__ __forceinline__ double gamma_q0(double v, double s, const GammaShape& g) {
+  return exp((log(v) + g.lg1) / s);
+}
+
+// The quantile and dx/ds.  It starts from the cubic interpolation of ln x
+// over ln(-ln(1-v)) in the shape's table (k_ws_table; error below 1e-6, so
+// the first step is already below 1e-5 and the series is summed twice, the
+// derivative included, instead of 4 to 6 times), outside the table and where
+// the shape has none (s < kGamMin: ln x is too steep) from the small-x form,
+// which took 3 to 4 steps on average and as many as its wave's slowest lane
+// (k_diff_src 0.63 -> 0.28 ms per 4096 Pb+Pb events, with the shape's
+// constants from the table as well).
+__device__ inline void gamma_qf(double v, double s, const double* tab, double& x, double& dxds) {
+  if (!(v > 0.0)) {
+    x = 0.0;
+    dxds = 0.0;
+    return;
+  }
+  const GammaShape g{tab[0], tab[1], tab[2]};
+  double xx = 0.0;
+  const double y = (log(-log1p(-v)) - kGamLo) * kGamPer;
+  if (s >= kGamMin && y >= 1.0 && y < kGamTab - 2) {
+    const int i = (int)y;
+    const double f = y - i;
+    const double* t = tab + 3 + i;
+    xx = exp(-f * (f - 1.0) * (f - 2.0) / 6.0 * t[-1] + (f + 1.0) * (f - 1.0) * (f - 2.0) / 2.0 * t[0] -
+             (f + 1.0) * f * (f - 2.0) / 2.0 * t[1] + (f + 1.0) * f * (f - 1.0) / 6.0 * t[2]);
+  }
+  if (!(xx > 0.0 && xx < HUGE_VAL)) xx = gamma_q0(v, s, g);
+  x = gamma_q(v, s, g, xx);
   double dP = 0.0;
-  gamma_p(s, x, lg1, psi1, &dP);
-  const double pdf = exp(-x + (s - 1.0) * log(x) - lgs);
+  gamma_p(s, x, g.lg1, g.psi1, &dP);
+  const double pdf = exp(-x + (s - 1.0) * log(x) - g.lgs);
   dxds = -dP / pdf;
 }
 
@@ -223,7 +257,27 @@ __device__ __forceinline__ double diff_shape(int kind, double alpha, double kg) 
 // tab[kWsTabInt + 3 i ..]; {Z, Z_R, Z_a} after the quantiles.  A node's
 // integrals are a chain of 64 terms, four to six times over: with one lane
 // per term the kernel takes 14 us instead of 157.
-__global__ __launch_bounds__(256) void k_ws_table(double R, double a, const double2* gl, int ngl, double* tab) {
+// The blocks after those (kg > 0) take one lane per entry of the two shapes'
+// Gamma tables: at tab + kWsTabGam + kind * kGamLen the shape's constants,
+// then ln x at v = 1 - exp(-exp(kGamLo + i / kGamPer)).
+__global__ __launch_bounds__(256) void k_ws_table(double R, double a, const double2* gl, int ngl, double* tab,
+                                                  double alpha, double kg) {
+  if (blockIdx.x >= kWsTabBlocks) {
+    const int k = (blockIdx.x - kWsTabBlocks) * 256 + threadIdx.x, kind = k / kGamTab, j = k % kGamTab;
+    if (kind >= 2) return;
+    double* t = tab + kWsTabGam + kind * kGamLen;
+    const double s = diff_shape(kind ? kSrcPair : kSrcPartA, alpha, kg);
+    const GammaShape g = gamma_shape(s);
+    if (j == 0) {
+      t[0] = g.lg1;
+      t[1] = g.psi1;
+      t[2] = g.lgs;
+    }
+    if (s < kGamMin) return;
+    const double v = -expm1(-exp(kGamLo + j / kGamPer));
+    t[3 + j] = log(gamma_q(v, s, g, gamma_q0(v, s, g)));
+    return;
+  }
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (i >= kWsTab) return;
   const WsNorm z = ws_norm_wave(R, a, gl, ngl);
@@ -420,7 +474,7 @@ __global__ __launch_bounds__(256) void k_diff_src(DevCfg cfg, EvBufs buf, DiffBu
       const double v = u53(r.x, r.y);
       const double sh = diff_shape(s.w, alpha, kg);
       double q, dq;
-      gamma_qf(v, sh, q, dq);
+      gamma_qf(v, sh, d.wstab + kWsTabGam + (s.w == kSrcPair ? kGamLen : 0), q, dq);
       f = q / sh;
       dfds = dq / sh - q / (sh * sh);
       d.gam_v[(size_t)e * buf.src_cap + k] = v;
@@ -723,8 +777,8 @@ __global__ __launch_bounds__(256) void k_diff_chain(DevCfg cfg, EvBufs buf, Diff
 int launch_diff_topo(const DevCfg& cfg, const EvBufs& b, const DiffBufs& d, int nev, unsigned long long seed,
                      unsigned long long event0, double R0, double a0, void* stream) {
   const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
-  hipLaunchKernelGGL(k_ws_table, dim3((kWsTab + 3) / 4), dim3(256), 0, (hipStream_t)stream, R0, a0, d.gl, d.ngl,
-                     d.wstab);
+  hipLaunchKernelGGL(k_ws_table, dim3(kWsTabBlocks), dim3(256), 0, (hipStream_t)stream, R0, a0, d.gl, d.ngl, d.wstab,
+                     0.0, 0.0);
   hipLaunchKernelGGL(k_diff_topo, dim3(nev), dim3(64), 0, (hipStream_t)stream, cfg, b, d, key, event0, R0, a0);
   return (int)hipGetLastError();
 }
@@ -733,8 +787,9 @@ int launch_diff_forward_pre(const DevCfg& cfg, const EvBufs& b, const DiffBufs& 
                             unsigned long long event0, const double* theta, int fluct, void* stream) {
   const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_ws_table, dim3((kWsTab + 3) / 4), dim3(256), 0, st, theta[1], theta[2], d.gl, d.ngl,
-                     d.wstab);
+  const int gamma_blocks = fluct ? 2 * kGamTab / 256 : 0;
+  hipLaunchKernelGGL(k_ws_table, dim3(kWsTabBlocks + gamma_blocks), dim3(256), 0, st, theta[1], theta[2], d.gl, d.ngl,
+                     d.wstab, theta[3], theta[4]);
   hipLaunchKernelGGL(k_diff_pos, dim3(nev), dim3(256), 0, st, cfg, d, theta[1], theta[2]);
   hipLaunchKernelGGL(k_diff_src, dim3(nev), dim3(256), 0, st, cfg, b, d, key, event0, theta[3], theta[4], fluct);
   return (int)hipGetLastError();

@@ -136,13 +136,19 @@ struct DiffBufs {
   double* gev;        // [ev][5] dL/dtheta per event
   const double2* gl;  // Gauss-Legendre nodes/weights on [0, 1]: ngl, then kWsNear of a short rule
   int ngl;
-  double* wstab;      // [kWsTabLen] radial quantiles of the current (R, a), Z, Z_R, Z_a, the quantiles' N, N_R, N_a
+  double* wstab;      // [kWsTabLen] radial quantiles of the current (R, a), Z, Z_R, Z_a, the quantiles' N, N_R, N_a, the Gamma tables
   double* cotc;       // [ev][kCotStride] coefficients of the cell cotangents (k_diff_cot_coef)
 };
 constexpr int kCotStride = 12;  // c0, then (lam cx/S, lam cy/S, lam Ar/(Am N), lam Ai/(Am N), lam Am/N^2) for n = 2, 3
 constexpr int kWsTab = 2049;              // radial quantile nodes, uniform in u^(1/3)
 constexpr int kWsTabInt = kWsTab + 3;     // + the normalisation and its R, a derivatives
-constexpr int kWsTabLen = kWsTabInt + 3 * kWsTab;  // + N and its R, a derivatives at the nodes
+constexpr int kWsTabGam = kWsTabInt + 3 * kWsTab;  // + N and its R, a derivatives at the nodes
+constexpr int kWsTabBlocks = (kWsTab + 3) / 4;
+// Gamma quantile tables of the two shapes: entry i at -ln(1-v) = exp(kGamLo + i / kGamPer)
+constexpr int kGamTab = 512, kGamLen = 3 + kGamTab;
+constexpr double kGamLo = -8.0, kGamPer = (kGamTab - 1) / 11.2;  // up to 1 - v = 2e-11
+constexpr double kGamMin = 0.02;                                 // smallest shape with a table
+constexpr int kWsTabLen = kWsTabGam + 2 * kGamLen;
 constexpr int kWsNear = 6;                // nodes of the integral from the nearest table node
 // per-event scalars of the differentiable moments
 enum : int {

@@ -50,3 +50,25 @@ def test_repeated_calls_agree_to_the_bit():
                 first = out, g
             np.testing.assert_array_equal(out, first[0])
             np.testing.assert_array_equal(g, first[1])
+
+
+@pytest.mark.parametrize("k", [0.1, 0.8, 5.0, 30.0])
+def test_gamma_quantiles(k):
+    """Shapes with and without a quantile table (pairs at k = 0.1: 0.014) up
+    to 13: forward and gradient against FP64 at test_gpu_adjoint's bars."""
+    from supermc_amd import Context
+    nev = 2
+    with Context(H.glauber_params("PbPb", max_events=nev)) as ctx:
+        th = ctx.diff_setup(seed=21, event0=0, nev=nev)
+        evs = [D.event_from_context(ctx, e) for e in range(nev)]
+        th = np.array([*th[:4], k])
+        out = ctx.diff_forward(th)
+        g = ctx.diff_backward(np.tile(COT, (nev, 1)))
+        for e, ev in enumerate(evs):
+            ref = ev.forward(th)
+            assert abs(out[e, 0] - ref[0]) <= 1e-6 and abs(out[e, 1] - ref[1]) <= 1e-6
+            assert out[e, 2] == pytest.approx(ref[2], rel=1e-5)
+        ref = sum(ev.adjoint(th, COT) for ev in evs)
+        scale = np.abs(ref).max()
+        for q in range(5):
+            assert abs(g[q] - ref[q]) <= 1e-4 * max(abs(ref[q]), 1e-3 * scale), (q, g[q], ref[q])
