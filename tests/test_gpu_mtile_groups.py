@@ -11,7 +11,7 @@ import parity_helpers as H
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("A", [1, 3, 9, 17, 40])
+@pytest.mark.parametrize("A", [1, 5, 9, 17, 40])
 @pytest.mark.parametrize("path,bar", [(1, 1e-5), (4, 1e-5), (3, 1e-5 + 3 * 2.0 ** -16)])
 def test_groups_match_valu_tiles(A, path, bar):
     from supermc_amd import Context
