@@ -56,19 +56,25 @@ __global__ __launch_bounds__(256) void k_cm_angle(DevCfg cfg, EvBufs buf, const 
     const float* g = grid + (size_t)e * cfg.nx * cfg.ny;
     for (int ix = R.x0 + wv; ix < R.x1; ix += 4) {
       const double x = cfg.xmin + ix * cfg.dx - xc;
-      for (int iy = R.y0 + lane; iy < R.y1; iy += 64) {
-        const double d = (double)g[(size_t)ix * cfg.ny + iy];
-        if (d == 0.0) continue;
-        const double y = cfg.ymin + iy * cfg.dy - yc;
-        // r^n cos(n theta), r^n sin(n theta) = Re, Im (x + i y)^n
-        double zr = x, zi = y;
-        for (int k = 1; k < n; ++k) {
-          const double nr = zr * x - zi * y, ni = zr * y + zi * x;
-          zr = nr;
-          zi = ni;
+      for (int yb = R.y0 + lane; yb < R.y1; yb += 256) {
+        float v[4];  // four loads in flight, added in column order
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = yb + 64 * j < R.y1 ? g[(size_t)ix * cfg.ny + yb + 64 * j] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const double d = (double)v[j];
+          if (d == 0.0) continue;
+          const double y = cfg.ymin + (yb + 64 * j) * cfg.dy - yc;
+          // r^n cos(n theta), r^n sin(n theta) = Re, Im (x + i y)^n
+          double zr = x, zi = y;
+          for (int k = 1; k < n; ++k) {
+            const double nr = zr * x - zi * y, ni = zr * y + zi * x;
+            zr = nr;
+            zi = ni;
+          }
+          re += zr * d;
+          im += zi * d;
         }
-        re += zr * d;
-        im += zi * d;
       }
     }
   }
