@@ -529,41 +529,44 @@ __global__ __launch_bounds__(64) void k_diff_cot_coef(DiffBufs d, const double* 
 }
 
 // Cell cotangents G = dL/drho inside each event's source rectangle -- the
-// cells the gather reads (every source window lies in it); kCotBlocks
-// workgroups per event stride over the rectangle's cells.
-constexpr int kCotBlocks = 64;
+// cells the gather reads (every source window lies in it); the waves of
+// kCotBlocks workgroups per event stride over the rectangle's rows (one cell
+// index for all of it cost a 64-bit division per cell: 0.32 -> 0.20 ms per 4096 Pb+Pb events).
+constexpr int kCotBlocks = 16;
 __global__ __launch_bounds__(256) void k_diff_cot(DevCfg cfg, EvBufs buf, DiffBufs d, float* G) {
   __shared__ double cf[kCotStride];
-  const int e = blockIdx.y;
+  const int e = blockIdx.y, lane = threadIdx.x & 63;
   const int nx = cfg.nx, ny = cfg.ny, nwy = (ny + 31) >> 5;
   const double* sc = d.dsc + (size_t)e * kDsStride;
   if (threadIdx.x < kCotStride) cf[threadIdx.x] = d.cotc[(size_t)e * kCotStride + threadIdx.x];
   __syncthreads();
   const int rx = buf.counts[(size_t)e * 8 + 6], ry = buf.counts[(size_t)e * 8 + 7];
   const int x0 = rx & 0xffff, x1 = rx >> 16, y0 = ry & 0xffff, y1 = ry >> 16;
-  const int wy = y1 - y0;
-  const size_t ncr = (x1 > x0 && wy > 0) ? (size_t)(x1 - x0) * wy : 0;
   const double c0 = cf[0], ax = cf[1] + cf[6], ay = cf[2] + cf[7];
   const double xc = sc[kDsXc], yc = sc[kDsYc];
   const bool third = cf[8] != 0.0 || cf[9] != 0.0 || cf[10] != 0.0;
-  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < ncr; k += (size_t)kCotBlocks * blockDim.x) {
-    const int ix = x0 + (int)(k / wy), iy = y0 + (int)(k % wy);
-    const double x = cfg.xmin + ix * cfg.dx - xc, y = cfg.ymin + iy * cfg.dy - yc;
-    const double r2 = x * x + y * y;
-    const bool m = (d.mask[(size_t)e * nx * nwy + (size_t)ix * nwy + (iy >> 5)] >> (iy & 31)) & 1u;
-    double g = c0;
-    g += ax * x + ay * y;
-    if (m && r2 > 0.0) {
-      // g_n(z) = z^n r^(2-n)
-      const double gr = x * x - y * y, gi = 2.0 * x * y;
-      g += cf[3] * gr + cf[4] * gi - cf[5] * r2;
-      if (third) {
-        const double ir = 1.0 / sqrt(r2);
-        const double tr = (gr * x - gi * y) * ir, ti = (gr * y + gi * x) * ir;
-        g += cf[8] * tr + cf[9] * ti - cf[10] * r2;
+  const int wave = 4 * blockIdx.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int ix = x0 + wave; ix < x1; ix += 4 * kCotBlocks) {
+    const unsigned* mrow = d.mask + ((size_t)e * nx + ix) * nwy;
+    float* row = G + ((size_t)e * nx + ix) * ny;
+    for (int iy = y0 + lane; iy < y1; iy += 64) {
+      const double x = cfg.xmin + ix * cfg.dx - xc, y = cfg.ymin + iy * cfg.dy - yc;
+      const double r2 = x * x + y * y;
+      const bool m = (mrow[iy >> 5] >> (iy & 31)) & 1u;
+      double g = c0;
+      g += ax * x + ay * y;
+      if (m && r2 > 0.0) {
+        // g_n(z) = z^n r^(2-n)
+        const double gr = x * x - y * y, gi = 2.0 * x * y;
+        g += cf[3] * gr + cf[4] * gi - cf[5] * r2;
+        if (third) {
+          const double ir = 1.0 / sqrt(r2);
+          const double tr = (gr * x - gi * y) * ir, ti = (gr * y + gi * x) * ir;
+          g += cf[8] * tr + cf[9] * ti - cf[10] * r2;
+        }
       }
+      row[iy] = (float)g;
     }
-    G[(size_t)e * nx * ny + (size_t)ix * ny + iy] = (float)g;
   }
 }
 
