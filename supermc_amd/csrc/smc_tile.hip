@@ -743,8 +743,15 @@ int tile_units(const DevCfg& cfg) { return ((cfg.nx + kTileRows - 1) / kTileRows
 //                   1000 167 / 198 / 725
 static int waves_of(const DevCfg& cfg, const SmearSpec& s, int nev) {
   constexpr int kWaves[kTileVariants] = {0, 1, 4, 16};
-  if (cfg.tile_variant > 0 && cfg.tile_variant < kTileVariants) return kWaves[cfg.tile_variant];
   const long long tiles = (long long)tile_units(cfg) * nev;
+  if (cfg.tile_variant > 0 && cfg.tile_variant < kTileVariants) {
+    // a launch has fewer than 2^32 work-items: batches beyond that for the
+    // variant's shape (93,000 events of 45 tiles with sixteen waves) take the
+    // next smaller one; one wave per tile fits any batch that memory holds
+    int waves = kWaves[cfg.tile_variant];
+    while (waves > 1 && (tiles + 8 * tile_units(cfg)) * 64 * waves >= (1LL << 32)) waves /= 4;
+    return waves;
+  }
   const bool pairs = s.enabled[kSrcPair];
   return tiles <= (pairs ? 9000 : 2200) ? 16 : (tiles <= (pairs ? 58000 : 20000) ? 4 : 1);
 }
