@@ -28,10 +28,11 @@
 //
 // The exact cut bounds the kernel.  It took a branch, two LDS reads and their
 // wait for every flagged patch of every source; with a source's 12 factors
-// read together, the four patches of a row taken without branches and the
-// sources without flags skipped by a ballot, 12,000 mixed events of 521^2
-// cells take 6.6 ms instead of 10.4 (BF16x3), and with the LDS of half a
-// group, 16 waves instead of 11 on a CU, 5.5 ms; grids bit-identical.
+// read together, the patches of a row taken without branches and the sources
+// without flags skipped by a ballot, 12,000 mixed events of 521^2 cells take
+// 6.6 ms instead of 10.4 (BF16x3); with the LDS of half a group, 16 waves
+// instead of 11 on a CU, 5.5 ms; with a branch per pair of patches instead of
+// per row of four, 5.3 ms.  Grids bit-identical.
 //
 // Precision (PREC):
 //   0  FP32: v_mfma_f32_16x16x4_f32, 4 sources per instruction;
@@ -174,10 +175,10 @@ __global__ __launch_bounds__(64, EPI == 0 && PREC != 0 ? 5 - PREC : 1) void k_mt
     }
     return bits;
   };
-  // Exact cut of the pass's source s: subtract, in the rows of patches of mask
-  // mk, the products that the MFMA adds outside the disk.  Every factor that
-  // the source can need is read first (12 reads in flight), and the patches
-  // of a row are taken together: a branch for each costs as much as a patch.
+  // Exact cut of the pass's source s: subtract, in the pairs of patches that
+  // mask mk flags, the products that the MFMA adds outside the disk.  Every
+  // factor that the source can need is read first (12 reads in flight); a
+  // branch for each patch costs as much as the patch.
   auto cut = [&](int s, unsigned mk, float wsb) {
     float gx[8], gy[4];
 #pragma unroll
@@ -185,12 +186,12 @@ __global__ __launch_bounds__(64, EPI == 0 && PREC != 0 ? 5 - PREC : 1) void k_mt
 #pragma unroll
     for (int r = 0; r < 8; ++r) gx[r] = la[r >> 2][4 * (r & 3) + q][s];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      if (!((mk >> (4 * r)) & 15u)) continue;
+    for (int r = 0; r < 16; ++r) {
+      if (!((mk >> (2 * r)) & 3u)) continue;
 #pragma unroll
-      for (int ci = 0; ci < 4; ++ci) {
-        const float t = gx[r] * gy[ci];
-        acc[r >> 2][ci][r & 3] -= (t < thr) ? t * wsb : 0.f;
+      for (int ci = 2 * (r & 1); ci < 2 * (r & 1) + 2; ++ci) {
+        const float t = gx[r >> 1] * gy[ci];
+        acc[r >> 3][ci][(r >> 1) & 3] -= (t < thr) ? t * wsb : 0.f;
       }
     }
   };
