@@ -230,8 +230,8 @@ def time_config1(nev, steps, seed):
                k_grid64_write_gbps=nev * N * 8 / (k64 * 1e-3) / 1e9,
                grid_bytes_per_event={"fp32": N * 4, "fp64": N * 8},
                note="*_grids_events_per_s: wall time incl. the device-to-host copies of every grid (pinned); "
-                    "device_events_per_s_*: kernel time with the grids left in HBM; k_grid64 evaluates exp per "
-                    "(source, window cell) in FP64, FP64 VALU bound")
+                    "device_events_per_s_*: kernel time with the grids left in HBM; k_grid64 adds one FP64 term per "
+                    "(source, window cell), FP64 VALU bound")
     return out
 
 
@@ -239,10 +239,9 @@ def time_kln_direct(nev, steps, seed):
     """MC-KLN Pb+Pb with dN/dy from the k_T-factorised quadrature in every
     cell (kln_direct = 1): 32 pT x 32 kT x 48 phi Gauss-Legendre nodes, phi
     and 2 pi - phi merged, so 32 x 768 node terms per cell with T_A, T_B > 0.
-    The work unit is the integrand's node term c min(1, a u) min(1, b v)
-    added to the sum, 5 flops as written (four multiplies and the add); the
-    kernel evaluates it as c min(1/a, u) min(1/b, v) with a b taken out per
-    pT node (two minima, a multiply and an FMA)."""
+    The kernel evaluates the node sum from tables of its values at the
+    breakpoints (bilinear in between): one 16-byte table entry per (cell,
+    pT node), so its rate is that of table bytes."""
     from supermc_amd import Context
     p = kln_params(nev)
     p.kln_direct = 1
@@ -260,12 +259,11 @@ def time_kln_direct(nev, steps, seed):
         active = float((s > 0).sum())
         nodes = p.kln_n_pt * p.kln_n_kt * (p.kln_n_phi // 2)
     kms = ms / max(n, 1)
-    tf = 5.0 * active * nodes / (kms * 1e-3) / 1e12
+    gbps = 16.0 * active * p.kln_n_pt / (kms * 1e-3) / 1e9
     return dict(events_per_s=nev * steps / dt, events_per_step=nev, steps=steps, k_kln_direct_ms=kms,
                 active_cells_per_event=active / nev, node_terms_per_cell=nodes,
-                roofline=dict(bound="valu", achieved_tflops=tf, frac=tf * 1e12 / FP32_PEAK,
-                              frac_nonpacked=tf * 1e12 / FP32_PEAK_NONPACKED,
-                              work="5 flops per (cell with T_A, T_B > 0, node)"))
+                roofline=dict(bound="hbm", achieved_gbps=gbps, frac=gbps * 1e9 / HBM_PEAK,
+                              work="16 table bytes per (cell with T_A, T_B > 0, pT node), cache hits included"))
 
 
 def _cpu_kln_worker(args):
