@@ -199,12 +199,12 @@ __device__ __forceinline__ TileEntry tile_entry(const DevCfg& cfg, const SmearSp
 // acc_sel only.
 //
 // What the kernels below do with the sums of rows r0 .. r0 + TR - 1 (lane =
-// column; aA: T_A where there are two): the epilogue, the stores, and per
-// column the sums p of each 8 rows for the centre-of-mass partials.
+// column; aA: T_A where there are two): the epilogue and the stores; the stored
+// values are left in a.
 template <int TR, int EPI>
 __device__ __forceinline__ void tile_finish(const DevCfg& cfg, const EvBufs& buf, const TileAt& at, int r0, bool live,
                                             float (&a)[TR], const float (&aA)[EPI ? TR : 1], const KlnTab& kt,
-                                            float* out, double (&p)[TR / 8][2]) {
+                                            float* out) {
   constexpr bool TWO = EPI != 0;
   const int lane = threadIdx.x & 63, col = at.c0 + lane, nx = cfg.nx, ny = cfg.ny;
   const float so = cfg.tile_out;
@@ -226,13 +226,25 @@ __device__ __forceinline__ void tile_finish(const DevCfg& cfg, const EvBufs& buf
   float* o = out + (size_t)at.e * N + (size_t)r0 * ny + col;
 #pragma unroll
   for (int r = 0; r < TR; ++r) {
-    if (r % 8 == 0) p[r / 8][0] = p[r / 8][1] = 0.0;
-    if (col < ny && r0 + r < nx) {
-      const float f = a[r] * os;
-      o[(size_t)r * ny] = f;
-      const double v = (double)f;
-      p[r / 8][0] += v;
-      p[r / 8][1] = fma(cfg.xmin + (r0 + r) * cfg.dx, v, p[r / 8][1]);
+    a[r] *= os;
+    if (col < ny && r0 + r < nx) o[(size_t)r * ny] = a[r];
+  }
+}
+
+// Adds the stored values of rows r0 .. r0 + TR - 1 to the column sums s0 =
+// sum v and s1 = sum x v, in row order whatever the shape: the centre of mass
+// is the same to the bit, and with it what is ill-conditioned in it (the
+// order-1 angle of an averaged profile is one of rounding).
+template <int TR>
+__device__ __forceinline__ void column_sums(const DevCfg& cfg, const TileAt& at, int r0, const float (&a)[TR],
+                                            double& s0, double& s1) {
+  const int col = at.c0 + (threadIdx.x & 63);
+#pragma unroll
+  for (int r = 0; r < TR; ++r) {
+    if (col < cfg.ny && r0 + r < cfg.nx) {
+      const double v = (double)a[r];
+      s0 += v;
+      s1 = fma(cfg.xmin + (r0 + r) * cfg.dx, v, s1);
     }
   }
 }
@@ -384,15 +396,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EPI ? 1 : 7,
       if constexpr (TWO) aA[4 * i + j] = accA[i][j];
     }
   }
-  double p[TR / 8][2];
-  tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out, p);
+  tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out);
   if (spec.cm_out) {
-    double s0 = p[0][0], s1 = p[0][1];
-#pragma unroll
-    for (int h = 1; h < TR / 8; ++h) {
-      s0 += p[h][0];
-      s1 += p[h][1];
-    }
+    double s0 = 0.0, s1 = 0.0;
+    column_sums<TR>(cfg, at, r0, a, s0, s1);
     tile_cm(cfg, at, s0, s1, spec.cm_out);
   }
 }
@@ -411,7 +418,7 @@ __global__ __launch_bounds__(256) void k_tile4(DevCfg cfg, EvBufs buf, SmearSpec
   __shared__ float fx_s[2][kGB4][kTileRows];  // K gx: row 8 v + q + 4 i at 8 v + 2 q + i
   __shared__ float4 fy_s[2][kGB4][16];        // gy: column c + 16 k at 4 c + k
   __shared__ int cnt_s[NW];
-  __shared__ double cm_s[NW][2][64];
+  __shared__ double cm_s[2][64];
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), q = lane >> 4, c = lane & 15;
   const TileAt at = tile_at(cfg, buf, nev, spread, order);
   if (at.e < 0) return;
@@ -542,19 +549,17 @@ __global__ __launch_bounds__(256) void k_tile4(DevCfg cfg, EvBufs buf, SmearSpec
       if constexpr (TWO) aA[4 * i + j] = accA[i][j];
     }
   }
-  double p[1][2];
-  tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out, p);
+  tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out);
   if (!spec.cm_out) return;
-  cm_s[wv][0][lane] = p[0][0];
-  cm_s[wv][1][lane] = p[0][1];
-  __syncthreads();
-  if (wv == 0) {
-    double s0 = p[0][0], s1 = p[0][1];
-    for (int v = 1; v < NW; ++v) {
-      s0 += cm_s[v][0][lane];
-      s1 += cm_s[v][1][lane];
+  for (int v = 0; v < NW; ++v) {  // each wave goes on from the sums of the rows before its own
+    if (wv == v) {
+      double s0 = v ? cm_s[0][lane] : 0.0, s1 = v ? cm_s[1][lane] : 0.0;
+      column_sums<TR>(cfg, at, r0, a, s0, s1);
+      cm_s[0][lane] = s0;
+      cm_s[1][lane] = s1;
+      if (v == NW - 1) tile_cm(cfg, at, s0, s1, spec.cm_out);
     }
-    tile_cm(cfg, at, s0, s1, spec.cm_out);
+    __syncthreads();
   }
 }
 
@@ -601,7 +606,7 @@ __global__ __launch_bounds__(1024) void k_tile16(DevCfg cfg, EvBufs buf, SmearSp
   __shared__ float fy_s[2][kGB][64];         // gy
   __shared__ int cnt_s[NW];
   __shared__ float sum_s[TWO ? 2 : 1][kTileRows][64];
-  __shared__ double cm_s[4][2][64];
+  __shared__ double cm_s[2][64];
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), q = lane >> 4, c = lane & 15;
   const int wr = wv >> 2, wc = wv & 3;  // the wave's 8 rows and 16 columns: unit 4 wr + wc = wv
   const TileAt at = tile_at(cfg, buf, nev, spread, order);
@@ -706,28 +711,27 @@ __global__ __launch_bounds__(1024) void k_tile16(DevCfg cfg, EvBufs buf, SmearSp
     sum_s[TWO ? pass : 0][TR * wr + q + 4][16 * wc + c] = acc1;
   }
   __syncthreads();
+  const int r0 = R0 + TR * wv;
+  float a[TR] = {};
   if (wv < 4) {  // wave v stores rows 8 v .. 8 v + 7
-    const int r0 = R0 + TR * wv;
-    float a[TR], aA[TWO ? TR : 1];
+    float aA[TWO ? TR : 1];
 #pragma unroll
     for (int r = 0; r < TR; ++r) {
       a[r] = sum_s[TWO ? 1 : 0][TR * wv + r][lane];
       if constexpr (TWO) aA[r] = sum_s[0][TR * wv + r][lane];
     }
-    double p[1][2];
-    tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out, p);
-    cm_s[wv][0][lane] = p[0][0];
-    cm_s[wv][1][lane] = p[0][1];
+    tile_finish<TR, EPI>(cfg, buf, at, r0, live, a, aA, kt, out);
   }
   if (!spec.cm_out) return;
-  __syncthreads();
-  if (wv == 0) {
-    double s0 = cm_s[0][0][lane], s1 = cm_s[0][1][lane];
-    for (int v = 1; v < 4; ++v) {
-      s0 += cm_s[v][0][lane];
-      s1 += cm_s[v][1][lane];
+  for (int v = 0; v < 4; ++v) {  // as in k_tile4
+    if (wv == v) {
+      double s0 = v ? cm_s[0][lane] : 0.0, s1 = v ? cm_s[1][lane] : 0.0;
+      column_sums<TR>(cfg, at, r0, a, s0, s1);
+      cm_s[0][lane] = s0;
+      cm_s[1][lane] = s1;
+      if (v == 3) tile_cm(cfg, at, s0, s1, spec.cm_out);
     }
-    tile_cm(cfg, at, s0, s1, spec.cm_out);
+    __syncthreads();
   }
 }
 
