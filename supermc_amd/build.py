@@ -73,6 +73,17 @@ def build_facade():
     return lib, exe
 
 
+def build_checks():
+    """tests/native: programs that run parts of the host code on the CPU."""
+    src = os.path.join(ROOT, "tests", "native", "copy_check.cpp")
+    if os.path.exists(src):
+        out = os.path.join(ROOT, "tests", "native", "copy_check.bin")
+        rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+        _run([CXX, "-O2", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"), src,
+              os.path.join(CSRC, "smc_copy.cpp"), "-pthread", "-o", out + ".tmp"])
+        os.replace(out + ".tmp", out)
+
+
 def build(verbose=True):
     os.makedirs(LIBDIR, exist_ok=True)
     objs = []
@@ -93,6 +104,7 @@ def build(verbose=True):
     for o in objs:
         os.remove(o)
     build_facade()
+    build_checks()
     return out
 
 

@@ -103,7 +103,7 @@ hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_
 void parallel_memcpy(void* dst, const void* src, size_t bytes) {
   constexpr size_t kPiece = (size_t)1 << 20;
   const int n = bytes < (size_t)4 << 20 ? 1 : workers_for(bytes / kPiece);
-  const size_t per = (bytes / n + 4095) & ~(size_t)4095;
+  const size_t per = ((bytes + n - 1) / n + 4095) & ~(size_t)4095;  // n pieces of whole pages cover all bytes
   run_workers(n, [&](int i) {
     const size_t off = std::min(bytes, per * i), m = std::min(per, bytes - off);
     if (m) std::memcpy((char*)dst + off, (const char*)src + off, m);

@@ -1,0 +1,80 @@
+// copy_check.cpp -- smc_copy.cpp on the CPU: the check named on the command
+// line, 0 if it holds.  The HIP calls it makes are defined here, over host
+// memory: transfers are done when they are queued.
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "../../supermc_amd/csrc/smc_copy.h"
+
+extern "C" {
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  *p = std::malloc(n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = (hipEvent_t)std::malloc(1);
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+  std::free((void*)e);
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t*, const void*) { return hipErrorInvalidValue; }
+}
+
+namespace {
+
+int fail(const char* what, size_t at) {
+  std::fprintf(stderr, "%s (%zu)\n", what, at);
+  return 1;
+}
+
+std::vector<unsigned char> pattern(size_t n) {
+  std::vector<unsigned char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = (unsigned char)(1 + i % 251);
+  return v;
+}
+
+// every byte arrives, none past the end is written: counts around whole
+// pages per worker for any number of workers, and the smallest
+int check_memcpy() {
+  const auto src = pattern((size_t)17 << 20);
+  std::vector<unsigned char> dst(src.size());
+  for (size_t mib : {0, 4, 5, 6, 7, 8, 12, 16})
+    for (int r = mib ? -9 : 0; r <= 9; ++r) {
+      const size_t n = (mib << 20) + r;
+      std::fill(dst.begin(), dst.begin() + n + 64, 0);
+      smc::parallel_memcpy(dst.data(), src.data(), n);
+      if (std::memcmp(dst.data(), src.data(), n) != 0) return fail("bytes missing", n);
+      for (size_t i = n; i < n + 64; ++i)
+        if (dst[i]) return fail("written past the end", n);
+    }
+  return 0;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const char* name = argc > 1 ? argv[1] : "";
+  if (!std::strcmp(name, "memcpy")) return check_memcpy();
+  return fail("no such check", 0);
+}

@@ -1,0 +1,14 @@
+"""The host side of the copies into ordinary memory (smc_copy.cpp), by a
+program that runs it on the CPU (native/copy_check.cpp)."""
+import os
+import subprocess
+
+import pytest
+
+CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "copy_check.bin")
+
+
+@pytest.mark.parametrize("name", ["memcpy"])
+def test_copies(name):
+    r = subprocess.run([CHECK, name], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
