@@ -13,6 +13,8 @@
  * doubles {x, y, eta, sigma_x, sigma_y, sigma_eta} (participant_info).
  * Grids are float [nev][grid_neta][grid_nx][grid_ny] (rho[j][k][l] of the
  * reference, y contiguous).
+ *
+ * Threads may share a handle: calls on it take turns.
  */
 #ifndef SMC_P3D_H
 #define SMC_P3D_H

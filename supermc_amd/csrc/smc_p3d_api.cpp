@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -29,6 +30,7 @@ struct smc_p3d {
   float* grid = nullptr;
   size_t grid_floats = 0;
   HostCopier copier;
+  std::mutex calls;  // the buffers above serve one call at a time
 };
 constexpr size_t kP3dGridBytes = (size_t)256 << 20;
 
@@ -263,6 +265,7 @@ smc_status smc_p3d_sample(smc_p3d* h, int nev, const double* part_xy, const int*
                           double* part_src, double* bin_src) {
   if (!h || nev < 0) return SMC_ERR_ARG;
   if (nev == 0) return SMC_OK;
+  const std::lock_guard<std::mutex> turn(h->calls);
   try {
     const Sources src = sample_dev(h, nev, part_xy, part_id, part_off, bin_xy, bin_off, seed, event0);
     if (part_src && src.np)
@@ -277,6 +280,7 @@ smc_status smc_p3d_sample(smc_p3d* h, int nev, const double* part_xy, const int*
 smc_status smc_p3d_smear(smc_p3d* h, int nev, const double* src, const int* src_off, float* rho) {
   if (!h || nev < 0 || !rho) return SMC_ERR_ARG;
   if (nev == 0) return SMC_OK;
+  const std::lock_guard<std::mutex> turn(h->calls);
   try {
     const int n = check_offsets(src_off, nev, "sources");
     if (n && !src) throw P3dError(SMC_ERR_ARG, "source records missing");
@@ -298,6 +302,7 @@ smc_status smc_p3d_generate(smc_p3d* h, int nev, const double* part_xy, const in
                             float* rho_part, float* rho_binary, double* part_src, double* bin_src) {
   if (!h || nev < 0) return SMC_ERR_ARG;
   if (nev == 0) return SMC_OK;
+  const std::lock_guard<std::mutex> turn(h->calls);
   try {
     const Sources src = sample_dev(h, nev, part_xy, part_id, part_off, bin_xy, bin_off, seed, event0);
     if (rho_part) grids_to_host(h, nev, src.part, src.part_off, rho_part);
