@@ -5,9 +5,7 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace smc {
 
@@ -18,24 +16,22 @@ int workers_for(size_t pieces) {
   return (int)std::min<size_t>(pieces, (size_t)std::max(1, std::min(HostCopier::kWorkers, hc / 2)));
 }
 
-// f(0) .. f(n - 1) at once, f(0) on this thread; where a thread cannot be
-// started, on this one
+// f(0) .. f(n - 1) at once, n <= kWorkers, f(0) on this thread; where a thread
+// cannot be started (no thread, no memory), on this one
 template <class F>
-void run_workers(int n, const F& f) {
-  std::vector<std::thread> th;
-  std::vector<int> left;
-  th.reserve(n);
-  left.reserve(n);
+void run_workers(int n, const F& f) noexcept {
+  std::thread th[HostCopier::kWorkers];
   for (int i = 1; i < n; ++i) {
     try {
-      th.emplace_back(f, i);
-    } catch (const std::system_error&) {
-      left.push_back(i);
+      th[i] = std::thread(f, i);
+    } catch (...) {
     }
   }
   f(0);
-  for (int i : left) f(i);
-  for (auto& t : th) t.join();
+  for (int i = 1; i < n; ++i)
+    if (!th[i].joinable()) f(i);
+  for (int i = 1; i < n; ++i)
+    if (th[i].joinable()) th[i].join();
 }
 
 }  // namespace

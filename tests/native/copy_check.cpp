@@ -5,9 +5,21 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "../../supermc_amd/csrc/smc_copy.h"
+
+// allocations left before one fails (negative: none fails)
+static thread_local int g_allocations = -1;
+
+void* operator new(size_t n) {
+  if (g_allocations >= 0 && g_allocations-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipGetLastError() { return hipSuccess; }
@@ -71,10 +83,30 @@ int check_memcpy() {
   return 0;
 }
 
+// the bytes arrive, and no exception leaves the call, when any one of its
+// allocations (a thread's state) fails
+int check_allocations() {
+  const auto src = pattern((size_t)8 << 20);
+  std::vector<unsigned char> dst(src.size());
+  for (int k = 0; k < 2 * smc::HostCopier::kWorkers; ++k) {
+    std::fill(dst.begin(), dst.end(), 0);
+    try {
+      g_allocations = k;
+      smc::parallel_memcpy(dst.data(), src.data(), src.size());
+    } catch (...) {
+      return fail("exception", k);
+    }
+    g_allocations = -1;
+    if (dst != src) return fail("bytes missing", k);
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* name = argc > 1 ? argv[1] : "";
   if (!std::strcmp(name, "memcpy")) return check_memcpy();
+  if (!std::strcmp(name, "allocations")) return check_allocations();
   return fail("no such check", 0);
 }
