@@ -43,6 +43,16 @@ HostCopier::~HostCopier() {
   }
 }
 
+// worker i's slot and event; where either cannot be had, no error is left behind
+bool HostCopier::reserve(int i) {
+  if (!slot_[i] && hipHostMalloc(&slot_[i], kSlotBytes, hipHostMallocDefault) != hipSuccess) slot_[i] = nullptr;
+  if (slot_[i] && !done_[i] && hipEventCreateWithFlags(&done_[i], hipEventDisableTiming) != hipSuccess)
+    done_[i] = nullptr;
+  if (slot_[i] && done_[i]) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 bool HostCopier::staged(const void* dst, size_t bytes) {
   if (bytes < kStagedBytes) return false;
   hipPointerAttribute_t at{};
@@ -54,24 +64,21 @@ bool HostCopier::staged(const void* dst, size_t bytes) {
 }
 
 hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_t stream) {
-  if (!staged(dst, bytes)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
   const size_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
-  const int n = workers_for(pieces);
-  int dev = 0;
-  hipError_t rc = hipGetDevice(&dev);
-  for (int i = 0; i < n && rc == hipSuccess; ++i) {
-    if (!slot_[i]) rc = hipHostMalloc(&slot_[i], kSlotBytes, hipHostMallocDefault);
-    if (rc == hipSuccess && !done_[i]) rc = hipEventCreateWithFlags(&done_[i], hipEventDisableTiming);
+  int n = 0, dev = 0, of_stream = -1;  // n workers have a slot and an event
+  if (staged(dst, bytes)) {
+    if (hipGetDevice(&dev) == hipSuccess && hipStreamGetDevice(stream, &of_stream) == hipSuccess) {
+      while (of_stream == dev && n < workers_for(pieces) && reserve(n)) ++n;
+    } else {
+      (void)hipGetLastError();
+    }
   }
-  if (rc != hipSuccess) return rc;
+  if (n == 0) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
   std::mutex order;  // pieces are queued in the order they are taken
   const auto work = [&](int i) {
-    if (hipSetDevice(dev) != hipSuccess) {
-      err = (int)hipErrorInvalidDevice;
-      return;
-    }
+    if (i > 0 && hipSetDevice(dev) != hipSuccess) return;  // the pieces are left to the others
     while (err.load() == (int)hipSuccess) {
       size_t off, m;
       hipError_t e;

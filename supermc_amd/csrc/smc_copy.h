@@ -12,8 +12,9 @@ namespace smc {
 // the other workers' transfers run.  One thread through the runtime's own
 // staging reaches 10 GB/s on untouched pages (17 on touched ones); a
 // transfer into pinned memory runs at 57 GB/s and eight threads write 67 GB/s
-// to untouched pages.  Smaller copies and pinned destinations take one
-// hipMemcpyAsync.
+// to untouched pages.  Smaller copies, pinned destinations, a stream of
+// another device than the thread's, and copies for which no slot can be had
+// take one hipMemcpyAsync; with some of the slots there are fewer workers.
 //
 // One object per context or handle; not thread-safe, like them.  The slots
 // (at most kWorkers of them) are allocated by the first staged copy and freed
@@ -38,6 +39,7 @@ class HostCopier {
   static bool staged(const void* dst, size_t bytes);
 
  private:
+  bool reserve(int i);
   void* slot_[kWorkers] = {};
   hipEvent_t done_[kWorkers] = {};
 };

@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -21,30 +22,57 @@ void* operator new(size_t n) {
 void operator delete(void* p) noexcept { std::free(p); }
 void operator delete(void* p, size_t) noexcept { std::free(p); }
 
+// calls left before the kind fails from then on (negative: it does not fail)
+static int g_slots = -1, g_events = -1, g_device = -1, g_threads = -1;
+static hipError_t g_last = hipSuccess;
+static int g_stream_device = 0;
+
+static hipError_t after(int& left, hipError_t e) {
+  if (left < 0 || left-- > 0) return hipSuccess;
+  left = 0;
+  return g_last = e;
+}
+
 extern "C" {
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
 hipError_t hipGetDevice(int* d) {
   *d = 0;
+  return after(g_device, hipErrorNoDevice);
+}
+hipError_t hipSetDevice(int) {
+  static std::mutex one;
+  const std::lock_guard<std::mutex> g(one);
+  return after(g_threads, hipErrorInvalidDevice);
+}
+hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t* d) {
+  *d = g_stream_device;
   return hipSuccess;
 }
-hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
-  *p = std::malloc(n);
-  return hipSuccess;
+  const hipError_t e = after(g_slots, hipErrorOutOfMemory);
+  if (e == hipSuccess) *p = std::malloc(n);
+  return e;
 }
 hipError_t hipHostFree(void* p) {
   std::free(p);
   return hipSuccess;
 }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
-  *e = (hipEvent_t)std::malloc(1);
-  return hipSuccess;
+hipError_t hipEventCreateWithFlags(hipEvent_t* p, unsigned) {
+  const hipError_t e = after(g_events, hipErrorOutOfMemory);
+  if (e == hipSuccess) *p = (hipEvent_t)std::malloc(1);
+  return e;
 }
 hipError_t hipEventDestroy(hipEvent_t e) {
   std::free((void*)e);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) {
+  return g_stream_device == 0 ? hipSuccess : hipErrorInvalidHandle;  // events are of device 0
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
   std::memcpy(d, s, n);
@@ -102,11 +130,38 @@ int check_allocations() {
   return 0;
 }
 
+// a staged copy succeeds and leaves no error behind when the k-th and every
+// later slot, event, device query or worker's device call fails
+int check_slots() {
+  const auto src = pattern(((size_t)19 << 20) + 5);
+  std::vector<unsigned char> dst(src.size());
+  for (int* left : {&g_slots, &g_events, &g_device, &g_threads})
+    for (int k = 0; k < smc::HostCopier::kWorkers; ++k) {
+      smc::HostCopier copier;
+      for (int again = 0; again < 2; ++again) {  // the second call after the first could not get everything
+        std::fill(dst.begin(), dst.end(), 0);
+        *left = k;
+        const hipError_t e = copier.copy(dst.data(), src.data(), src.size(), nullptr);
+        *left = -1;
+        if (e != hipSuccess) return fail("error returned", k);
+        if (dst != src) return fail("bytes missing", k);
+        if (left != &g_threads && hipGetLastError() != hipSuccess) return fail("error left behind", k);
+      }
+    }
+  smc::HostCopier copier;
+  g_stream_device = 1;
+  std::fill(dst.begin(), dst.end(), 0);
+  if (copier.copy(dst.data(), src.data(), src.size(), nullptr) != hipSuccess || dst != src)
+    return fail("stream of another device", 1);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* name = argc > 1 ? argv[1] : "";
   if (!std::strcmp(name, "memcpy")) return check_memcpy();
   if (!std::strcmp(name, "allocations")) return check_allocations();
+  if (!std::strcmp(name, "slots")) return check_slots();
   return fail("no such check", 0);
 }
