@@ -74,14 +74,18 @@ def build_facade():
 
 
 def build_checks():
-    """tests/native: programs that run parts of the host code on the CPU."""
-    src = os.path.join(ROOT, "tests", "native", "copy_check.cpp")
-    if os.path.exists(src):
-        out = os.path.join(ROOT, "tests", "native", "copy_check.bin")
-        rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
-        _run([CXX, "-O2", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"), src,
-              os.path.join(CSRC, "smc_copy.cpp"), "-pthread", "-o", out + ".tmp"])
-        os.replace(out + ".tmp", out)
+    """tests/native: a program that runs host code on the CPU, and a
+    library that stands before the HIP runtime in a test process."""
+    native = os.path.join(ROOT, "tests", "native")
+    if not os.path.isdir(native):
+        return
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    for out, args in (("copy_check.bin", ["copy_check.cpp", os.path.join(CSRC, "smc_copy.cpp"), "-pthread"]),
+                      ("hip_refuse.so", ["hip_refuse.cpp", "-fPIC", "-shared"])):
+        tmp = os.path.join(native, out + ".tmp")
+        _run([CXX, "-O2", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"),
+              os.path.join(native, args[0]), *args[1:], "-o", tmp])
+        os.replace(tmp, os.path.join(native, out))
 
 
 def build(verbose=True):

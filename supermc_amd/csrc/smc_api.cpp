@@ -197,7 +197,8 @@ struct smc_ctx {
   unsigned* kln_list = nullptr;   // active cells of the per-cell quadrature (an event chunk), then its count
   int kln_npt = 0, kln_nn = 0;
   KlnConst kln_kc{};
-  KlnBreaks kln_breaks{};         // breakpoint tables of the per-cell quadrature (first use)
+  KlnBreaks kln_breaks{};         // breakpoint tables of the per-cell quadrature
+  int kln_breaks_done = 0;        // built, or the memory was refused (first use)
   // differentiable batches
   DiffBufs dif{};
   void* dif_alloc[16] = {};
@@ -742,23 +743,43 @@ void ensure_kln_table(smc_ctx* c) {
   (void)hipFree(db);
 }
 
-// The breakpoint tables of the per-cell quadrature, built on its first use;
-// node tables they do not fit stay on the node-by-node kernel.
+// Device memory, or null (and no error left behind) where it cannot be had.
+template <class T>
+T* try_dalloc(size_t n) {
+  void* p = nullptr;
+  if (hipMalloc(&p, n * sizeof(T)) == hipSuccess) return (T*)p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+// The breakpoint tables of the per-cell quadrature, built on its first use.
+// Node tables they do not fit, and contexts that cannot have the memory (151
+// MB at 32 x 768 nodes, up to 512 MiB), stay on the node-by-node kernel.  That
+// is settled once per context: the two kernels round differently, and a later
+// call may be a captured one.
 void ensure_kln_breaks(smc_ctx* c) {
-  KlnBreaks& kb = c->kln_breaks;
-  if (kb.tab || !kln_breaks_fit(c->kln_npt, c->kln_nn)) return;
+  if (c->kln_breaks_done || !kln_breaks_fit(c->kln_npt, c->kln_nn)) return;
   const size_t nb = (size_t)c->kln_npt * (c->kln_nn + 1);
-  if (!kb.bu) kb.bu = dalloc<float>(nb);
-  if (!kb.bv) kb.bv = dalloc<float>(nb);
-  if (!kb.sorted) kb.sorted = dalloc<double>(4 * (size_t)c->kln_npt * c->kln_nn);
-  float* tab = dalloc<float>(2 * kln_breaks_doubles(c->kln_npt, c->kln_nn));
-  kb.tab = tab;
-  const int rc = launch_kln_breaks(c->kln_nodes_d, c->kln_npt, c->kln_nn, kb, c->stream);
-  if (rc) {
-    kb.tab = nullptr;
-    (void)hipFree(tab);
-    check_launch(rc, "k_kln_breaks");
+  KlnBreaks kb{};
+  kb.tab = try_dalloc<float>(2 * kln_breaks_doubles(c->kln_npt, c->kln_nn));
+  if (kb.tab) kb.sorted = try_dalloc<double>(4 * (size_t)c->kln_npt * c->kln_nn);
+  if (kb.sorted) kb.bu = try_dalloc<float>(nb);
+  if (kb.bu) kb.bv = try_dalloc<float>(nb);
+  int rc = 0;
+  if (kb.bv) {
+    rc = launch_kln_breaks(c->kln_nodes_d, c->kln_npt, c->kln_nn, kb, c->stream);
+    if (!rc) rc = (int)hipStreamSynchronize(c->stream);
   }
+  if (kb.sorted) (void)hipFree(kb.sorted);
+  kb.sorted = nullptr;
+  if (!kb.bv || rc) {
+    for (void* p : {(void*)kb.bu, (void*)kb.bv, kb.tab})
+      if (p) (void)hipFree(p);
+    kb = KlnBreaks{};
+  }
+  check_launch(rc, "k_kln_breaks");
+  c->kln_breaks = kb;
+  c->kln_breaks_done = 1;
 }
 
 // MCnucl::setDensity for which_mc_model 1 (MCnucl.cpp:654-687): T_A, T_B
@@ -1383,7 +1404,7 @@ void smc_destroy(smc_ctx* c) {
                   c->buf.bval, c->buf.evkey, c->buf.order, c->buf.raw, c->buf.src, c->buf.swin, c->dtab, c->grid, c->ta, c->tb, c->tmp, c->evout,
                   c->cm, c->band, c->mrects, c->nmrect, c->avg_rot, c->avg_acc, c->avg_sum, c->avg_part, c->avg_ext, c->aux0,
                   c->aux1, c->grid64, c->spec_src, c->spec_swin, c->spec_counts, c->kln_table, c->kln_ptf, c->kln_nodes_f, c->kln_ptd, c->kln_nodes_d, c->kln_list,
-                  c->kln_breaks.bu, c->kln_breaks.bv, c->kln_breaks.sorted, c->kln_breaks.tab};
+                  c->kln_breaks.bu, c->kln_breaks.bv, c->kln_breaks.tab};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   for (void* q : c->dif_alloc)

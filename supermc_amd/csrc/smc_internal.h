@@ -292,7 +292,7 @@ int launch_diff_moments(const DevCfg& cfg, const EvBufs& b, const DiffBufs& d, c
 int launch_diff_backward(const DevCfg& cfg, const EvBufs& b, const SmearSpec& spec, const DiffBufs& d, int nev,
                          const double* cot_dev, double ffdxdy, float* G, const double* theta, void* stream);
 // breakpoint tables of the per-cell quadrature (smc_kln_direct.hip): bu, bv
-// [npt][nn + 1] floats, sorted [npt][nn] double4 (build only), tab
+// [npt][nn + 1] floats, sorted [npt][nn] double4 (while they are built), tab
 // kln_breaks_doubles() float2; all null: the node-by-node kernel
 struct KlnBreaks {
   float* bu;
