@@ -223,9 +223,10 @@ smc_status smc_density(smc_ctx* ctx, float* s, double* dndy);
 /* MCnucl::setDensity(iy=0, ipt=-1) in the reference's own precision: the
  * double grids of MCnucl.cpp:689-760 (which_mc_model 5) and :762-811 (7).
  * Every (source, cell) term is evaluated in FP64 on the cells the reference
- * takes (Particle.cpp:122-132, 168-174) and added in its order; the
- * exponential is the product of its row and column factors, a few ulp from
- * the reference's.
+ * takes (Particle.cpp:122-132, 168-174) and added in its order, participants
+ * and pairs in sums of their own; the exponential is the product of its row
+ * and column factors.  The rounding against exact sums is that of the
+ * reference's expressions or smaller, the last bits differ.
  * Events [ev0, ev0 + n) of the current batch; s host [n][nx][ny].
  * SMC_ERR_UNSUPPORTED for other models, SMC_ERR_ARG for a range outside
  * the batch. */

@@ -1691,6 +1691,7 @@ smc_status smc_density_f64(smc_ctx* c, int ev0, int n, double* s) {
     const double w = c->d.width, wsq = w * w;
     Grid64Const gc{};
     gc.norm = 1 / (2 * M_PI * w * w);
+    gc.norm_lo = (double)(1 / (2 * 3.14159265358979323846L * w * w) - gc.norm);
     gc.two_w_w = 2 * w * w;
     // the largest double whose root is at most 5 w (sqrt rounds monotonically)
     const double r_max = 5 * w;

@@ -182,7 +182,7 @@ struct SmearSpec {
 // FP64 density grids (smc_grid64.hip); constants computed on the host as the
 // reference writes them
 struct Grid64Const {
-  double norm;       // 1 / (2 pi w w)
+  double norm, norm_lo;  // 1 / (2 pi w w) and what its rounding left
   double two_w_w;    // 2 w w   (Particle.cpp:122-132, MCnucl.cpp:732-756)
   double part_max;   // the largest d^2 with sqrt(d^2) <= 5 w
   double dc_max;     // 25 (w w)
