@@ -37,6 +37,8 @@
 // slots of 6,700 in 8-row chunks of 64 columns remain for a 51-cell window.  At the end the 4 x 4 blocks (q, k) are
 // transposed across the lane groups, and a lane holds one column again:
 // stores of 64 consecutive cells.
+#include <algorithm>
+
 #include "smc_device.h"
 
 namespace smc {
@@ -737,14 +739,35 @@ __global__ __launch_bounds__(1024) void k_tile16(DevCfg cfg, EvBufs buf, SmearSp
 
 int tile_units(const DevCfg& cfg) { return ((cfg.nx + kTileRows - 1) / kTileRows) * ((cfg.ny + 63) / 64); }
 
+// About how many sources a central event's list holds: the nucleons that n
+// collisions wound and, where the spec has the pairs, the n pairs; n = 1.5 A B
+// sigma / (pi R^2) of the larger radius (a sphere is 1.5 times as thick at its
+// centre as on average).  Pb+Pb 3,400 with pairs and 416 without, 63+63 810
+// and 126, 20+20 170 and 40, d+Au 60 and 30, p+Pb 30 and 15.  The nuclei are
+// the context's, the largest of a mixed batch.
+static double central_list(const DevCfg& cfg, const SmearSpec& s) {
+  const NucSys &p = cfg.nuc[0], &t = cfg.nuc[1];
+  const double R = std::max(1.0, (double)std::max(p.R, t.R));
+  const double n = std::min((double)p.A * t.A, 1.5 * p.A * t.A * (double)cfg.hit_n * (kQ * kQ) / (R * R));
+  return std::min((double)p.A, n) + std::min((double)t.A, n) + (s.enabled[kSrcPair] ? n : 0.0);
+}
+
 // Waves per tile.  Variants 1, 2, 3 (smc_set_tile_variant) are one, four and
-// sixteen; 0 chooses by the number of tiles and by whether the lists hold the
-// collision pairs (a central Pb+Pb list is then 2,000 sources long, else 400).
-// Per batch of Pb+Pb events of 261^2 cells (45 tiles), us with 1 / 4 / 16 waves:
-//   with pairs      1 event 282 / 141 / 72, 128 472 / 239 / 145, 256 482 / 243 / 261,
+// sixteen; 0 chooses by the number of tiles and the length of a central list.
+// us with 1 / 4 / 16 waves per batch of events of 261^2 cells (45 tiles):
+//   Pb+Pb, pairs    1 event 282 / 141 / 72, 128 472 / 239 / 145, 256 482 / 243 / 261,
 //                   1000 504 / 362 / 1013, 2000 560 / 694 / 2018
-//   MC-KLN, sqrt    1 event 67 / 33 / 20, 64 95 / 48 / 63, 512 106 / 111 / 389,
+//   Pb+Pb, MC-KLN   1 event 67 / 33 / 20, 64 95 / 48 / 63, 512 106 / 111 / 389,
 //                   1000 167 / 198 / 725
+//   20+20, pairs    30 events 38 / 26 / 23, 200 44 / 28 / 72, 500 48 / 44 / 158,
+//                   1000 50 / 71 / 300
+//   p+Pb, pairs     8 events 17 / 12 / 11, 200 24 / 22 / 59, 500 30 / 36 / 133,
+//                   1000 39 / 58 / 255
+//   p+Pb, MC-KLN    8 events 26 / 15 / 15, 200 37 / 29 / 82, 500 47 / 49 / 188,
+//                   1000 70 / 81 / 359
+// A short list leaves sixteen waves nothing but their barriers.
+constexpr double kShortList = 100.0, kLongList = 700.0;
+
 static int waves_of(const DevCfg& cfg, const SmearSpec& s, int nev) {
   constexpr int kWaves[kTileVariants] = {0, 1, 4, 16};
   const long long tiles = (long long)tile_units(cfg) * nev;
@@ -756,21 +779,27 @@ static int waves_of(const DevCfg& cfg, const SmearSpec& s, int nev) {
     while (waves > 1 && (tiles + 8 * tile_units(cfg)) * 64 * waves >= (1LL << 32)) waves /= 4;
     return waves;
   }
-  const bool pairs = s.enabled[kSrcPair];
-  return tiles <= (pairs ? 9000 : 2200) ? 16 : (tiles <= (pairs ? 58000 : 20000) ? 4 : 1);
+  const double list = central_list(cfg, s);
+  if (list < kShortList) return tiles <= 9000 ? 4 : 1;
+  const bool heavy = list >= kLongList;
+  return tiles <= (heavy ? 9000 : 2200) ? 16 : (tiles <= (heavy ? 58000 : 20000) ? 4 : 1);
 }
 
-// Longest events first: 1000 events 735 -> 504 us with one wave per tile, 543 ->
-// 362 with four; 16,000 events 3.2 -> 2.9 ms.  One workgroup orders 32,768
-// events in about 60 us; larger batches lose less to their last tiles.
-static bool ordered(int nev) { return nev >= 16 && nev <= 32768; }
+// Longest events first: 1000 Pb+Pb events 735 -> 504 us with one wave per tile,
+// 543 -> 362 with four; 16,000 events 3.2 -> 2.9 ms.  One workgroup orders
+// 32,768 events in about 60 us; larger batches lose less to their last tiles.
+// Events of short lists are too alike to gain it back (p+Pb: 5 of 25 us at 200
+// events, 60 of 470 at 20,000).
+static bool ordered(const DevCfg& cfg, const SmearSpec& s, int nev) {
+  return nev >= 16 && nev <= 32768 && central_list(cfg, s) >= kShortList;
+}
 
 template <int EPI>
 static void launch_shape(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int acc_sel, int nev, float* out,
                          const KlnTab& kt, hipStream_t st) {
   const int waves = waves_of(cfg, s, nev);
   const int spread = nev < 64;  // 8 events per XCD keep its 32 CUs busy
-  const int* order = ordered(nev) ? b.order : nullptr;
+  const int* order = ordered(cfg, s, nev) ? b.order : nullptr;
   // one dimension: tiles x events; with an event's tiles on one XCD, events
   // padded to a multiple of the 8 XCDs
   const dim3 grid((unsigned)tile_units(cfg) * (spread ? (unsigned)nev : (unsigned)((nev + 7) / 8 * 8)));
@@ -782,8 +811,9 @@ static void launch_shape(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s,
     hipLaunchKernelGGL(k_tile<EPI>, grid, dim3(64), 0, st, cfg, b, s, acc_sel, nev, spread, order, out, kt);
 }
 
-static void launch_order(const EvBufs& b, int nev, hipStream_t st) {
-  if (ordered(nev)) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, st, b.counts, nev, 2048, b.order);
+static void launch_order(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev, hipStream_t st) {
+  if (ordered(cfg, s, nev))
+    hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, st, b.counts, nev, 2048, b.order);
 }
 
 // The fused MC-KLN launch (its centre-of-mass partials have tile_units(cfg)
@@ -793,7 +823,7 @@ int launch_tile_kln(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int 
   if (nev <= 0) return 0;
   if (!(cfg.tile_k > 0.f && cfg.tile_w > 0.f && cfg.tile_out > 0.f) || !table || tmax < 3 || !(dT > 0))
     return (int)hipErrorInvalidValue;
-  launch_order(b, nev, (hipStream_t)stream);
+  launch_order(cfg, b, s, nev, (hipStream_t)stream);
   launch_shape<1>(cfg, b, s, 0, nev, out, KlnTab{table, tmax, dT}, (hipStream_t)stream);
   return (int)hipGetLastError();
 }
@@ -826,7 +856,7 @@ int launch_tile(const DevCfg& cfg, const EvBufs& b, const SmearSpec& s, int nev,
   if (!(cfg.tile_k > 0.f && cfg.tile_w > 0.f && cfg.tile_out > 0.f)) return (int)hipErrorInvalidValue;
   hipStream_t st = (hipStream_t)stream;
   const KlnTab none{nullptr, 0, 1.0};
-  launch_order(b, nev, st);
+  launch_order(cfg, b, s, nev, st);
   if (s.combine == 1) {  // sqrt(T_A T_B) in one launch, with the partials of the combined grid
     launch_shape<2>(cfg, b, s, 0, nev, out0, none, st);
     return (int)hipGetLastError();
