@@ -37,20 +37,31 @@ void run_workers(int n, const F& f) noexcept {
 }  // namespace
 
 HostCopier::~HostCopier() {
-  for (int i = 0; i < kWorkers; ++i) {
-    if (done_[i]) (void)hipEventDestroy(done_[i]);
-    if (slot_[i]) (void)hipHostFree(slot_[i]);
-  }
+  for (hipEvent_t e : done_)
+    if (e) (void)hipEventDestroy(e);
+  if (slots_) (void)hipHostFree(slots_);
 }
 
-// worker i's slot and event; where either cannot be had, no error is left behind
-bool HostCopier::reserve(int i) {
-  if (!slot_[i] && hipHostMalloc(&slot_[i], kSlotBytes, hipHostMallocDefault) != hipSuccess) slot_[i] = nullptr;
-  if (slot_[i] && !done_[i] && hipEventCreateWithFlags(&done_[i], hipEventDisableTiming) != hipSuccess)
-    done_[i] = nullptr;
-  if (slot_[i] && done_[i]) return true;
-  (void)hipGetLastError();
-  return false;
+// How many of n workers have a slot and an event for a copy of these bytes;
+// where they cannot be had, no error is left behind.
+int HostCopier::reserve(int n, size_t bytes) {
+  if (!slots_) {
+    seen_ += bytes;
+    if (seen_ < kSlotsFromBytes) return 0;
+    seen_ = 0;
+    if (hipHostMalloc((void**)&slots_, kWorkers * kSlotBytes, hipHostMallocDefault) != hipSuccess) {
+      slots_ = nullptr;
+      (void)hipGetLastError();
+      return 0;
+    }
+  }
+  for (int i = 0; i < n; ++i)
+    if (!done_[i] && hipEventCreateWithFlags(&done_[i], hipEventDisableTiming) != hipSuccess) {
+      done_[i] = nullptr;
+      (void)hipGetLastError();
+      return i;
+    }
+  return n;
 }
 
 bool HostCopier::staged(const void* dst, size_t bytes) {
@@ -68,7 +79,7 @@ hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_
   int n = 0, dev = 0, of_stream = -1;  // n workers have a slot and an event
   if (staged(dst, bytes)) {
     if (hipGetDevice(&dev) == hipSuccess && hipStreamGetDevice(stream, &of_stream) == hipSuccess) {
-      while (of_stream == dev && n < workers_for(pieces) && reserve(n)) ++n;
+      if (of_stream == dev) n = reserve(workers_for(pieces), bytes);
     } else {
       (void)hipGetLastError();
     }
@@ -79,6 +90,7 @@ hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_
   std::mutex order;  // pieces are queued in the order they are taken
   const auto work = [&](int i) {
     if (i > 0 && hipSetDevice(dev) != hipSuccess) return;  // the pieces are left to the others
+    char* const slot = slots_ + (size_t)i * kSlotBytes;
     while (err.load() == (int)hipSuccess) {
       size_t off, m;
       hipError_t e;
@@ -88,7 +100,7 @@ hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_
         if (p >= pieces) return;
         off = p * kSlotBytes;
         m = std::min(kSlotBytes, bytes - off);
-        e = hipMemcpyAsync(slot_[i], (const char*)src + off, m, hipMemcpyDeviceToHost, stream);
+        e = hipMemcpyAsync(slot, (const char*)src + off, m, hipMemcpyDeviceToHost, stream);
         if (e == hipSuccess) e = hipEventRecord(done_[i], stream);
       }
       if (e == hipSuccess) e = hipEventSynchronize(done_[i]);
@@ -96,7 +108,7 @@ hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_
         err = (int)e;
         return;
       }
-      std::memcpy((char*)dst + off, slot_[i], m);
+      std::memcpy((char*)dst + off, slot, m);
     }
   };
   run_workers(n, work);

@@ -7,23 +7,27 @@
 namespace smc {
 
 // Copies of at least kStagedBytes into pageable memory go through pinned
-// slots, one per worker thread: each worker takes the next kSlotBytes piece,
+// slots (once there are slots, below), one per worker thread: each worker takes the next kSlotBytes piece,
 // queues its transfer into its slot and moves it on to the destination while
 // the other workers' transfers run.  One thread through the runtime's own
 // staging reaches 10 GB/s on untouched pages (17 on touched ones); a
 // transfer into pinned memory runs at 57 GB/s and eight threads write 67 GB/s
 // to untouched pages.  Smaller copies, pinned destinations, a stream of
 // another device than the thread's, and copies for which no slot can be had
-// take one hipMemcpyAsync; with some of the slots there are fewer workers.
+// take one hipMemcpyAsync.
 //
 // One object per context or handle; not thread-safe, like them.  The slots
-// (at most kWorkers of them) are allocated by the first staged copy and freed
-// with the object.
+// (one block for kWorkers of them, freed with the object) take 1.4 ms to make,
+// the time that they save on 8 MiB of untouched pages or 45 MiB of touched
+// ones: they are made for the copy that brings the object's bytes to
+// kSlotsFromBytes.  Made for the first 4 MiB, they had the first 20 FP64 grids
+// of a context (11 MB) take 2.4 ms instead of 1.7.
 class HostCopier {
  public:
   static constexpr int kWorkers = 8;
   static constexpr size_t kSlotBytes = (size_t)2 << 20;
   static constexpr size_t kStagedBytes = (size_t)4 << 20;
+  static constexpr size_t kSlotsFromBytes = (size_t)16 << 20;
 
   HostCopier() = default;
   HostCopier(const HostCopier&) = delete;
@@ -35,13 +39,14 @@ class HostCopier {
   // the stream has been waited for (a staged copy is complete on return).
   hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
 
-  // whether copy() would stage these bytes
+  // whether these bytes are worth staging, given the slots
   static bool staged(const void* dst, size_t bytes);
 
  private:
-  bool reserve(int i);
-  void* slot_[kWorkers] = {};
+  int reserve(int n, size_t bytes);
+  char* slots_ = nullptr;
   hipEvent_t done_[kWorkers] = {};
+  size_t seen_ = 0;  // bytes of copies worth staging, until there are slots
 };
 
 // memcpy by several threads where that pays

@@ -25,7 +25,7 @@ void operator delete(void* p, size_t) noexcept { std::free(p); }
 // calls left before the kind fails from then on (negative: it does not fail)
 static int g_slots = -1, g_events = -1, g_device = -1, g_threads = -1;
 static hipError_t g_last = hipSuccess;
-static int g_stream_device = 0;
+static int g_stream_device = 0, g_made = 0;
 
 static hipError_t after(int& left, hipError_t e) {
   if (left < 0 || left-- > 0) return hipSuccess;
@@ -53,6 +53,7 @@ hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t* d) {
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  ++g_made;
   const hipError_t e = after(g_slots, hipErrorOutOfMemory);
   if (e == hipSuccess) *p = std::malloc(n);
   return e;
@@ -156,6 +157,27 @@ int check_slots() {
   return 0;
 }
 
+// slots are made for the copy that brings a copier's bytes to
+// kSlotsFromBytes, at once for one that large, and once
+int check_first() {
+  const auto src = pattern((size_t)16 << 20);
+  std::vector<unsigned char> dst(src.size());
+  for (size_t mib : {3, 4, 5, 6, 8, 15, 16}) {
+    smc::HostCopier copier;
+    g_made = 0;
+    for (size_t total = 0; total < ((size_t)48 << 20);) {
+      const size_t n = mib << 20;
+      total += n;
+      std::fill(dst.begin(), dst.end(), 0);
+      if (copier.copy(dst.data(), src.data(), n, nullptr) != hipSuccess || std::memcmp(dst.data(), src.data(), n) != 0)
+        return fail("bytes missing", mib);
+      const bool due = n >= smc::HostCopier::kStagedBytes && total >= smc::HostCopier::kSlotsFromBytes;
+      if (g_made != (due ? 1 : 0)) return fail("slots made", mib);
+    }
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -163,5 +185,6 @@ int main(int argc, char** argv) {
   if (!std::strcmp(name, "memcpy")) return check_memcpy();
   if (!std::strcmp(name, "allocations")) return check_allocations();
   if (!std::strcmp(name, "slots")) return check_slots();
+  if (!std::strcmp(name, "first")) return check_first();
   return fail("no such check", 0);
 }

@@ -8,7 +8,7 @@ import pytest
 CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "copy_check.bin")
 
 
-@pytest.mark.parametrize("name", ["memcpy", "allocations", "slots"])
+@pytest.mark.parametrize("name", ["memcpy", "allocations", "slots", "first"])
 def test_copies(name):
     r = subprocess.run([CHECK, name], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
