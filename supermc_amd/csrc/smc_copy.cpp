@@ -1,8 +1,12 @@
 // smc_copy.cpp -- pageable device-to-host copies by worker threads (smc_copy.h)
 #include "smc_copy.h"
 
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <atomic>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -42,13 +46,26 @@ HostCopier::~HostCopier() {
   if (slots_) (void)hipHostFree(slots_);
 }
 
+// whether most pages of the destination have not been touched yet (four are
+// looked at)
+static bool untouched(const void* dst, size_t bytes) {
+  const size_t page = (size_t)sysconf(_SC_PAGESIZE);
+  int fresh = 0;
+  for (int i = 0; i < 4; ++i) {
+    const uintptr_t at = ((uintptr_t)dst + bytes / 8 * (2 * i + 1)) / page * page;
+    unsigned char in_memory = 1;
+    if (mincore((void*)at, page, &in_memory) == 0 && !(in_memory & 1)) ++fresh;
+  }
+  return fresh > 2;
+}
+
 // How many of n workers have a slot and an event for a copy of these bytes;
 // where they cannot be had, no error is left behind.
-int HostCopier::reserve(int n, size_t bytes) {
+int HostCopier::reserve(int n, const void* dst, size_t bytes) {
   if (!slots_) {
-    seen_ += bytes;
-    if (seen_ < kSlotsFromBytes) return 0;
-    seen_ = 0;
+    saved_us_ += (double)bytes / (1 << 20) * (untouched(dst, bytes) ? kFreshUs : kWrittenUs);
+    if (saved_us_ < kSlotsUs) return 0;
+    saved_us_ = 0;
     if (hipHostMalloc((void**)&slots_, kWorkers * kSlotBytes, hipHostMallocDefault) != hipSuccess) {
       slots_ = nullptr;
       (void)hipGetLastError();
@@ -79,7 +96,7 @@ hipError_t HostCopier::copy(void* dst, const void* src, size_t bytes, hipStream_
   int n = 0, dev = 0, of_stream = -1;  // n workers have a slot and an event
   if (staged(dst, bytes)) {
     if (hipGetDevice(&dev) == hipSuccess && hipStreamGetDevice(stream, &of_stream) == hipSuccess) {
-      if (of_stream == dev) n = reserve(workers_for(pieces), bytes);
+      if (of_stream == dev) n = reserve(workers_for(pieces), dst, bytes);
     } else {
       (void)hipGetLastError();
     }

@@ -18,16 +18,17 @@ namespace smc {
 //
 // One object per context or handle; not thread-safe, like them.  The slots
 // (one block for kWorkers of them, freed with the object) take 1.4 ms to make,
-// the time that they save on 8 MiB of untouched pages or 45 MiB of touched
-// ones: they are made for the copy that brings the object's bytes to
-// kSlotsFromBytes.  Made for the first 4 MiB, they had the first 20 FP64 grids
-// of a context (11 MB) take 2.4 ms instead of 1.7.
+// and a copy through them saves 185 us per MiB of a destination whose pages
+// are untouched and 32 us of one already written: they are made for the copy
+// with which the object's copies would have saved as much.  Made for the first
+// 4 MiB, they had the first 20 FP64 grids of a context (11 MB, written before)
+// take 2.4 ms instead of 1.7.
 class HostCopier {
  public:
   static constexpr int kWorkers = 8;
   static constexpr size_t kSlotBytes = (size_t)2 << 20;
   static constexpr size_t kStagedBytes = (size_t)4 << 20;
-  static constexpr size_t kSlotsFromBytes = (size_t)16 << 20;
+  static constexpr double kSlotsUs = 1400, kFreshUs = 185, kWrittenUs = 32;  // to make the slots; saved per MiB
 
   HostCopier() = default;
   HostCopier(const HostCopier&) = delete;
@@ -43,10 +44,10 @@ class HostCopier {
   static bool staged(const void* dst, size_t bytes);
 
  private:
-  int reserve(int n, size_t bytes);
+  int reserve(int n, const void* dst, size_t bytes);
   char* slots_ = nullptr;
   hipEvent_t done_[kWorkers] = {};
-  size_t seen_ = 0;  // bytes of copies worth staging, until there are slots
+  double saved_us_ = 0;  // what slots would have saved, until there are some
 };
 
 // memcpy by several threads where that pays

@@ -1,6 +1,8 @@
 // copy_check.cpp -- smc_copy.cpp on the CPU: the check named on the command
 // line, 0 if it holds.  The HIP calls it makes are defined here, over host
 // memory: transfers are done when they are queued.
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -131,10 +133,10 @@ int check_allocations() {
   return 0;
 }
 
-// a staged copy succeeds and leaves no error behind when the k-th and every
+// a large copy succeeds and leaves no error behind when the k-th and every
 // later slot, event, device query or worker's device call fails
 int check_slots() {
-  const auto src = pattern(((size_t)19 << 20) + 5);
+  const auto src = pattern(((size_t)45 << 20) + 5);
   std::vector<unsigned char> dst(src.size());
   for (int* left : {&g_slots, &g_events, &g_device, &g_threads})
     for (int k = 0; k < smc::HostCopier::kWorkers; ++k) {
@@ -157,24 +159,27 @@ int check_slots() {
   return 0;
 }
 
-// slots are made for the copy that brings a copier's bytes to
-// kSlotsFromBytes, at once for one that large, and once
+// Slots are made once, for the copy with which the copies so far would have
+// saved the time: after 44 MiB into written pages, 8 MiB into untouched ones.
 int check_first() {
   const auto src = pattern((size_t)16 << 20);
-  std::vector<unsigned char> dst(src.size());
-  for (size_t mib : {3, 4, 5, 6, 8, 15, 16}) {
-    smc::HostCopier copier;
-    g_made = 0;
-    for (size_t total = 0; total < ((size_t)48 << 20);) {
-      const size_t n = mib << 20;
-      total += n;
-      std::fill(dst.begin(), dst.end(), 0);
-      if (copier.copy(dst.data(), src.data(), n, nullptr) != hipSuccess || std::memcmp(dst.data(), src.data(), n) != 0)
-        return fail("bytes missing", mib);
-      const bool due = n >= smc::HostCopier::kStagedBytes && total >= smc::HostCopier::kSlotsFromBytes;
-      if (g_made != (due ? 1 : 0)) return fail("slots made", mib);
+  for (const bool fresh : {false, true})
+    for (size_t mib : {3, 4, 5, 6, 8, 15, 16}) {
+      smc::HostCopier copier;
+      g_made = 0;
+      double saved = 0;
+      for (int k = 0; k < 12; ++k) {
+        const size_t n = mib << 20;
+        char* dst = (char*)mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+        if (!fresh) std::memset(dst, 1, n);
+        if (copier.copy(dst, src.data(), n, nullptr) != hipSuccess || std::memcmp(dst, src.data(), n) != 0)
+          return fail("bytes missing", mib);
+        munmap(dst, n);
+        if (n >= smc::HostCopier::kStagedBytes)
+          saved += (double)mib * (fresh ? smc::HostCopier::kFreshUs : smc::HostCopier::kWrittenUs);
+        if (g_made != (saved >= smc::HostCopier::kSlotsUs ? 1 : 0)) return fail("slots made", mib);
+      }
     }
-  }
   return 0;
 }
 
