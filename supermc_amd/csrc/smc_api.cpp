@@ -629,7 +629,7 @@ SmearSpec density_spec(const smc_ctx* c) {
   if (c->p.which_mc_model == 5 && g.uli) {
     // MCnucl.cpp:713-717, 724-760 ("Ulrich" Glauber, sub_model 2): no
     // participant term; pair k adds f_k (alpha + (1 - alpha) aw_k) G, the
-    // product held in the pair's source weight (k_event)
+    // product held in the pair's source weight (k_sources)
     s.enabled[kSrcPair] = g.use_binary;
     s.win[kSrcPair] = kWin5;
     s.scale[kSrcPair] = g.norm;
@@ -669,11 +669,12 @@ SmearSpec thickness_spec(const smc_ctx* c) {
   return s;
 }
 
-// smear_path: 0 exact footprint on VALU tiles (k_tile: 32 x 64 by default,
-// one wave, disk cut by flushing denormal products); 1 the same footprint as
-// an FP32 MFMA contraction over the square window with the out-of-disk
-// products subtracted (k_mtile); 2 exact footprint, per-cell exponentials
-// (k_smear); 3 and 4 as 1 with BF16x3 and BF16x6 split-precision MFMA.
+// smear_path: 0 exact footprint on VALU tiles (k_tile, k_tile4, k_tile16: 32 x
+// 64 by 1, 4 or 16 waves, disk cut by flushing denormal products); 1 the same
+// footprint as an FP32 MFMA contraction over the square window with the
+// out-of-disk products subtracted (k_mtile); 2 exact footprint, per-cell
+// exponentials (k_smear); 3 and 4 as 1 with BF16x3 and BF16x6 split-precision
+// MFMA.
 // Every path takes every model and grid size.
 static int mfma_prec(const smc_ctx* c) {
   switch (c->p.smear_path) {

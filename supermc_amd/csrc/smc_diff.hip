@@ -5,7 +5,8 @@
 // and diffuseness (both nuclei), two-component mixing, Gamma k = 1/theta.
 // Frozen at theta0: the uniforms of every accepted nucleon, the impact
 // parameter, participants and collision pairs, every source's integer
-// footprint window with its r <= 5 w0 disk cut, and the hot-spot mask.
+// footprint window (in both directions the footprint is the whole window,
+// without the disk cut), and the hot-spot mask.
 //
 //  positions  r = F^{-1}(u; R, a), F the Woods-Saxon radial CDF truncated at
 //             R + 2.5 (the law of Nucleus.cpp:578-621), times a fixed unit
@@ -17,9 +18,9 @@
 //  density    the exact-footprint tile kernel with w in the Gaussian and the
 //             frozen windows.
 //  adjoint    cell cotangents G = dL/drho inside each event's source
-//             rectangle (k_diff_cot_coef, k_diff_cot), one wavefront per
-//             source gathering G against the recomputed Gaussians
-//             (k_diff_gather), per-event chain rule to theta (k_diff_chain).
+//             rectangle (k_diff_cot_coef, k_diff_cot), 16 lanes per source
+//             gathering G against the recomputed Gaussians (k_diff_gather),
+//             per-event chain rule to theta (k_diff_chain).
 #include "smc_device.h"
 
 namespace smc {
@@ -581,7 +582,8 @@ __global__ __launch_bounds__(256) void k_diff_cot(DevCfg cfg, EvBufs buf, DiffBu
 //   P = sum_r Ex_r g_rc,  Q = sum_r Ex_r dx_r g_rc,  R = sum_r Ex_r dx_r^2 g_rc,
 // folded with the column's Ey and dy at the end of a block of 64 rows:
 //   e0 = Ey P,  e1 = Ey Q,  e2 = Ey dy P,  e3 = Ey (R + dy^2 P).
-// VALU bound, so the layout is the one with the fewest instructions per cell:
+// Bound by VALU issue (0.255 instructions per SIMD and cycle, a chain of FMAs
+// reaches 0.245), so the layout is the one with the fewest per cell:
 // a wave takes four sources, 16 lanes each, and a lane 4 adjacent columns of
 // every row.  A row costs one 16-byte load and one 8-byte LDS read for 4
 // cells and 5 operations per cell (a lane per column took 10, with each row's

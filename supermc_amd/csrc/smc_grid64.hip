@@ -31,8 +31,10 @@
 // One workgroup of 4 waves per (32 x 64 tile, event), a wave 8 rows, laid out as
 // k_tile4 of smc_tile.hip: lane (q, c) holds rows q, q + 4 and columns c + 16 k;
 // the workgroup selects 256 sources at a time and shares the factors of 8.
-// Bound by the factors' exponentials and VALU issue about equally: 250 Au+Au
-// events of 261^2 cells 497 us (2226 us with an exponential per term).
+// 250 Au+Au events of 261^2 cells 497 us (2226 us with an exponential per term):
+// VALU instructions issue at 57 % of the rate of a chain of FMAs with 2.5 waves
+// on a SIMD, the rest is the waits between the factors' exponentials, LDS and
+// barriers.
 // Tiles outside the event's source rectangle are written as zeros without a
 // source pass.
 #include "smc_device.h"

@@ -251,9 +251,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         // held as z * 2^24, so d^2 < dmin^2 reads d2q < dmin^2 * 2^48.  Two
         // nucleons are that close only if every coordinate differs by less than
         // dmin: that is tested first, on float coordinates (each off by at
-        // most 16 quanta), and the distance only where some lane passes.  Five
-        // VALU instructions per pair instead of ten; this kernel is VALU bound
-        // (its VALU was busy 82 % of the time, two thirds of it in these
+        // most 32 quanta within 64 fm), and the distance only where some lane
+        // passes.  Five VALU instructions per pair instead of ten; this kernel is
+        // VALU bound (it was busy 82 % of the time, two thirds of it in these
         // pairs): 50,000 Pb+Pb events 4.20 -> 3.39 ms.
         const float dmin2q = cfg.dmin2 * 0x1p48f;
         const float near_q = sqrtf(cfg.dmin2) * (0x1p24f * 1.0001f) + 64.f;
@@ -625,8 +625,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
 // k_event has written, one workgroup per event.  Apart from k_event because
 // it needs neither its LDS nor its registers: its waves then fill the chip.
 // 50,000 Pb+Pb events: k_event 5.44 ms with this part, 4.21 without it and with
-// the shorter sorts, and 0.80 here, bound by the Gamma factors' logarithms and
-// powers and 1.1 GB of sources and windows written.
+// the shorter sorts, and 0.80 here: VALU instructions (the Gamma factors'
+// logarithms and powers) issue at 78 % of the rate of a chain of FMAs.
 __global__ __launch_bounds__(256) void k_sources(DevCfg cfg, EvBufs buf) {
   const int e = blockIdx.x, t = threadIdx.x, lane = t & 63;
   __shared__ int sx[2][kAMax], sy[2][kAMax];

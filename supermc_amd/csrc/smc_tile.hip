@@ -267,7 +267,8 @@ __device__ __forceinline__ void tile_cm(const DevCfg& cfg, const TileAt& at, dou
   }
 }
 
-// ---- one wave per tile, for batches that fill the chip: VALU issue bound (two
+// ---- one wave per tile, for batches that fill the chip: bound by VALU issue
+// (0.276 instructions per SIMD and cycle, a chain of FMAs reaches 0.245; two
 // instructions per cell slot, about 60 per source and tile around them).
 // 4 sources' factors in LDS at a time and 72 VGPRs (7 waves per SIMD): 8.93 ms
 // per 50,000 Pb+Pb events of 261^2 cells; 8 sources 9.45 (7 waves) and 9.41
@@ -755,10 +756,10 @@ static double central_list(const DevCfg& cfg, const SmearSpec& s) {
 // Waves per tile.  Variants 1, 2, 3 (smc_set_tile_variant) are one, four and
 // sixteen; 0 chooses by the number of tiles and the length of a central list.
 // us with 1 / 4 / 16 waves per batch of events of 261^2 cells (45 tiles):
-//   Pb+Pb, pairs    1 event 282 / 141 / 72, 128 472 / 239 / 145, 256 482 / 243 / 261,
-//                   1000 504 / 362 / 1013, 2000 560 / 694 / 2018
-//   Pb+Pb, MC-KLN   1 event 67 / 33 / 20, 64 95 / 48 / 63, 512 106 / 111 / 389,
-//                   1000 167 / 198 / 725
+//   Pb+Pb, pairs    30 events 404 / 196 / 105, 100 453 / 221 / 129, 200 468 / 225 / 233,
+//                   1000 514 / 342 / 1091, 2000 543 / 652 / 2168
+//   Pb+Pb, MC-KLN   30 events 89 / 47 / 40, 100 97 / 52 / 96, 500 105 / 109 / 401,
+//                   1000 163 / 191 / 768
 //   20+20, pairs    30 events 38 / 26 / 23, 200 44 / 28 / 72, 500 48 / 44 / 158,
 //                   1000 50 / 71 / 300
 //   p+Pb, pairs     8 events 17 / 12 / 11, 200 24 / 22 / 59, 500 30 / 36 / 133,
