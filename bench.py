@@ -231,7 +231,7 @@ def time_config1(nev, steps, seed):
                grid_bytes_per_event={"fp32": N * 4, "fp64": N * 8},
                note="*_grids_events_per_s: wall time incl. the device-to-host copies of every grid (pinned); "
                     "device_events_per_s_*: kernel time with the grids left in HBM; k_grid64 adds one FP64 term per "
-                    "(source, window cell), FP64 VALU bound")
+                    "(source, window cell); VALU issue at 57 % of a chain of FMAs")
     return out
 
 
@@ -240,8 +240,9 @@ def time_kln_direct(nev, steps, seed):
     cell (kln_direct = 1): 32 pT x 32 kT x 48 phi Gauss-Legendre nodes, phi
     and 2 pi - phi merged, so 32 x 768 node terms per cell with T_A, T_B > 0.
     The kernel evaluates the node sum from tables of its values at the
-    breakpoints (bilinear in between): one 16-byte table entry per (cell,
-    pT node), so its rate is that of table bytes."""
+    breakpoints (bilinear in between): a step, two searches and one 16-byte
+    table entry, per (cell, pT node).  It is bound by VALU issue, so the
+    table bytes, cache hits included, are a rate and not a share of HBM."""
     from supermc_amd import Context
     p = kln_params(nev)
     p.kln_direct = 1
@@ -259,11 +260,12 @@ def time_kln_direct(nev, steps, seed):
         active = float((s > 0).sum())
         nodes = p.kln_n_pt * p.kln_n_kt * (p.kln_n_phi // 2)
     kms = ms / max(n, 1)
-    gbps = 16.0 * active * p.kln_n_pt / (kms * 1e-3) / 1e9
+    per_s = active * p.kln_n_pt / (kms * 1e-3)
     return dict(events_per_s=nev * steps / dt, events_per_step=nev, steps=steps, k_kln_direct_ms=kms,
                 active_cells_per_event=active / nev, node_terms_per_cell=nodes,
-                roofline=dict(bound="hbm", achieved_gbps=gbps, frac=gbps * 1e9 / HBM_PEAK,
-                              work="16 table bytes per (cell with T_A, T_B > 0, pT node), cache hits included"))
+                roofline=dict(bound="valu", steps_per_s=per_s, table_gbps=16.0 * per_s / 1e9,
+                              work="one step per (cell with T_A, T_B > 0, pT node); 16 table bytes each, cache hits "
+                                   "included"))
 
 
 def _cpu_kln_worker(args):
