@@ -209,7 +209,7 @@ __global__ __launch_bounds__(64) void k_kln_breaks(const double4* __restrict__ s
 // searches run in step, so their LDS reads overlap (one search after the
 // other took 659 us at the size below, together 430 us).
 // Bound by VALU issue (0.243 instructions per SIMD and cycle, as many as a chain
-// of FMAs; the LDS is busy 14 % of the time).  150 Pb+Pb events of
+// of FMAs; a CU issues an LDS instruction every nine cycles).  150 Pb+Pb events of
 // 261^2 cells, 32 x 32 x 48 nodes: 430 us; summed node by node 3975 us
 // (four VALU per node term, 24,576 terms per cell).
 constexpr int KLN_R = 4;
