@@ -371,7 +371,8 @@ smc_status smc_get_event_system(smc_ctx* ctx, int ev, int* system);  /* -1: unmi
 
 /* Tile shapes of the exact-footprint smearing kernel (no counterpart in
  * the reference): 32 x 64 tiles with one (1), four (2) or sixteen (3) waves
- * each; 0 (default) chooses by the batch.  Every shape gives the same grids.
+ * each; 0 (default) chooses by the batch and its nuclei.  Every shape gives the
+ * same grids.
  * smc_autotune times each on the ctx's current events (reps launches after
  * a warm-up), keeps the fastest, and returns it with the per-shape times in
  * ms[SMC_TILE_VARIANTS] (either pointer may be NULL). */
