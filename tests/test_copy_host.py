@@ -10,5 +10,7 @@ CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "copy
 
 @pytest.mark.parametrize("name", ["memcpy", "allocations", "slots", "first"])
 def test_copies(name):
+    if not os.path.exists(CHECK):
+        pytest.fail(f"{CHECK} not built: run python -m supermc_amd.build")
     r = subprocess.run([CHECK, name], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr

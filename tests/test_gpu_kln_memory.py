@@ -50,6 +50,8 @@ def child():
 
 
 def test_density_without_memory_for_the_tables():
+    if not os.path.exists(os.path.join(HERE, "native", "hip_refuse.so")):
+        pytest.fail("tests/native/hip_refuse.so not built: run python -m supermc_amd.build")
     r = subprocess.run([sys.executable, os.path.abspath(__file__)], capture_output=True, text=True, timeout=110)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "without tables" in r.stdout
